@@ -67,7 +67,10 @@ int pa_tiled_fwd(const void* q, const void* k, const void* v, void* o, float* s,
 int pa_tiled_fwd_noalloc(const void* q, const void* k, const void* v, void* o,
                          int dtype, int64_t bh, int64_t n, int64_t d, int causal, void* stream);
 
-/* v3 fused: online softmax with fp32 arithmetic throughout (fp32 MFMA, P kept in fp32).
+/* v3 fused: online softmax with fp32 arithmetic throughout: fp32 inputs on the fp32 matrix core, P
+ * kept in fp32; fp16 inputs on the fp16 matrix core, whose products are exact, with P in two fp16
+ * terms of 22 significant bits (errors against float64 below the fp32 matrix core's). fp16 calls
+ * take fused_tc's launch forms, and pa_set_persistent() applies to them.
  * dtype: F32 or F16; out_dtype: dtype or F32; d == 64.
  * Replaces attn::launch_fused<T> (csrc/kernels/fused.cuh:106-112) and fused_forward
  * (csrc/attn_fused.cu:5-14). */
@@ -103,7 +106,7 @@ int pa_fused_tc_fwd(const void* q, const void* k, const void* v, void* o,
  * No reference counterpart: the reference launches one fixed kernel (csrc/kernels/fused_tc.cuh:187-196). */
 const char* pa_fused_tc_kernel(int dtype, int out_dtype, int64_t bh, int64_t n, int64_t d, int causal);
 
-/* Process-wide switch of fused_tc's persistent launch: enable = 0 selects one workgroup
+/* Process-wide switch of the persistent launch (fused_tc, and fused with fp16 inputs): enable = 0 selects one workgroup
  * per query block, nonzero the persistent launch. Returns the previous setting. The initial
  * setting is read once, when the library is loaded, from the environment variable
  * PA_PERSISTENT ("0" = off; unset or anything else = on). For A/B measurements and tests; calls

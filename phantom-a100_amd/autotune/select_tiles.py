@@ -78,9 +78,10 @@ def kernel_key(dtype: torch.dtype, d: int, br: int, bc: int, stages: int, out_dt
                ksplit: int = 1, persistent: bool = False, ragged: bool = False, causal: bool = False,
                check: bool = False) -> str:
     """Fragment of the mangled name of
-    pa::fa_mfma_fwd<T, D, BM, BN, STAGES, OutT, KSPLIT, PERSIST, RAGGED, CAUSAL, CHECK>."""
+    pa::fa_mfma_fwd<T, D, BM, BN, STAGES, OutT, KSPLIT, PERSIST, RAGGED, CAUSAL, CHECK, TERMS>, up
+    to CHECK (TERMS is 1 in every fused_tc and fused_tuned kernel)."""
     return (f"fa_mfma_fwdI{MANGLED_T[dtype]}Li{d}ELi{br}ELi{bc}ELi{stages}E{MANGLED_T[out_dtype]}"
-            f"Li{ksplit}ELb{int(persistent)}ELb{int(ragged)}ELb{int(causal)}ELb{int(check)}EE")
+            f"Li{ksplit}ELb{int(persistent)}ELb{int(ragged)}ELb{int(causal)}ELb{int(check)}E")
 
 
 def launch_form(entry: str, dtype: torch.dtype, d: int, n: int, bh: int, causal: bool, br: int,
@@ -121,7 +122,7 @@ def load_resources(path: str = RESOURCES) -> dict:
 
 def find_resources(res: dict, key: str) -> dict | None:
     for name, v in res.items():
-        if key in name:
+        if key in name and key + "Li2E" not in name:   # Li2E: `fused`'s two-term form of the same tile
             return dict(v, kernel=name)
     return None
 

@@ -1,9 +1,10 @@
-// Fused online-softmax attention forward with fp32 arithmetic throughout (the `fused` entry).
+// Fused online-softmax attention forward with fp32 arithmetic throughout (the `fused` entry's fp32
+// inputs; its fp16 inputs take fa_mfma.hpp's two-term form).
 //
 // Same algorithm and numerics as the reference's v3 kernel
 // (/root/reference/csrc/kernels/fused.cuh:26-102): Q pre-scaled by log2(e)/sqrt(d) in fp32
-// registers, scores, running max/sum and P all fp32 (P is never rounded), inputs fp32 or fp16
-// widened to fp32 on load. Both products run on the fp32 matrix core (v_mfma_f32_32x32x2_f32):
+// registers, scores, running max/sum and P all fp32 (P is never rounded). Both products run on
+// the fp32 matrix core (v_mfma_f32_32x32x2_f32):
 //   S^T (keys x queries) = K . Q^T   A = K (lane: one key row, 32 consecutive dims),
 //                                    B = scaled Q^T in VGPRs, k-slot h of step kk = dim h*D/2+kk
 //   O^T (d x queries)   += V^T . P^T  B = P^T straight from the S^T accumulator (k-slot h of
@@ -11,8 +12,7 @@
 //                                    the two keys of the step)
 // Each lane keeps all state of query l%32 (see fa_mfma.hpp). Row i of the two 32-row O^T blocks
 // is dim 2i (block 0) and dim 2i + 1 (block 1), so each lane reads the V values of both blocks
-// with one 8-byte load (fp32; 4 bytes for fp16) instead of two scalar loads; the merge puts the
-// dims back in order.
+// with one 8-byte load instead of two scalar loads; the merge puts the dims back in order.
 //
 // gfx950 shape: the fp32 matrix core does 64 FLOP per cycle per SIMD, so a 32-query x 32-key
 // tile costs a wave ~4K cycles; at the reference's sizes (N = 128) a wave per 32 queries leaves
@@ -35,62 +35,35 @@ struct F32Lds {
   static constexpr int BYTES = KS * 32 * (LDO + 2) * 4;
 };
 
-// 32 consecutive elements of a row, widened to fp32 (offsets past the buffer read as zero).
-// The loaded vector is bit-cast as a whole before its elements are taken: bit-casting an element
-// extracted from the u32x4 miscompiles with this toolchain (every element read as element 0).
-template <typename T>
+// 32 consecutive elements of a row (offsets past the buffer read as zero). The loaded vector is
+// bit-cast as a whole before its elements are taken: bit-casting an element extracted from the
+// u32x4 miscompiles with this toolchain (every element read as element 0).
 __device__ __forceinline__ void load_row32(rsrc_t rs, uint32_t byte_off, float (&x)[32]) {
-  if constexpr (sizeof(T) == 4) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const f32x4 w = __builtin_bit_cast(f32x4, load16(rs, byte_off + 16 * i));
+  for (int i = 0; i < 8; ++i) {
+    const f32x4 w = __builtin_bit_cast(f32x4, load16(rs, byte_off + 16 * i));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[4 * i + j] = w[j];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const u32x4 w = load16(rs, byte_off + 16 * i);
-      const f16x8 h = __builtin_bit_cast(f16x8, w);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[8 * i + j] = (float)h[j];
-    }
+    for (int j = 0; j < 4; ++j) x[4 * i + j] = w[j];
   }
 }
 
-template <typename T>
-__device__ __forceinline__ float load_one(rsrc_t rs, uint32_t byte_off) {
-  if constexpr (sizeof(T) == 4) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, byte_off, 0, 0));
-  } else {
-    return (float)__builtin_bit_cast(f16, __builtin_amdgcn_raw_buffer_load_b16(rs, byte_off, 0, 0));
-  }
-}
-
-// Two consecutive elements of a row, widened to fp32 (offsets past the buffer read as zero).
-template <typename T>
+// Two consecutive elements of a row (offsets past the buffer read as zero).
 __device__ __forceinline__ void load_pair(rsrc_t rs, uint32_t byte_off, float& a, float& b) {
-  if constexpr (sizeof(T) == 4) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    const f32x2 w = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, byte_off, 0, 0));
-    a = w[0];
-    b = w[1];
-  } else {
-    const f16x2 h = __builtin_bit_cast(f16x2, __builtin_amdgcn_raw_buffer_load_b32(rs, byte_off, 0, 0));
-    a = (float)h[0];
-    b = (float)h[1];
-  }
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  const f32x2 w = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, byte_off, 0, 0));
+  a = w[0];
+  b = w[1];
 }
 
-template <typename T, int D, int KS, typename OutT>
+template <int D, int KS>
 __global__ void __launch_bounds__(KS * kWave)
-fa_f32_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-           OutT* __restrict__ O, int N, int num_qblocks, int total_blocks, float scale_log2, int causal) {
+fa_f32_fwd(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+           float* __restrict__ O, int N, int num_qblocks, int total_blocks, float scale_log2, int causal) {
   typedef F32Lds<D, KS> L;
   constexpr int BN = 32;                     // keys per tile
   constexpr int NDB = D / 32;
   constexpr int HALF = D / 2;
-  constexpr int ES = sizeof(T);
+  constexpr int ES = sizeof(float);
   static_assert(D == 64, "the fp32 path is compiled for d = 64");
 
   __shared__ __attribute__((aligned(16))) float red_o[KS * 32 * L::LDO];
@@ -117,7 +90,7 @@ fa_f32_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict
 
   // Scaled Q^T operand: k-slot `hi` of step kk is dim hi*HALF + kk (rows past N read as zero).
   float qf[HALF];
-  load_row32<T>(q_rs, (uint32_t)((qrow * D + hi * HALF) * ES), qf);
+  load_row32(q_rs, (uint32_t)((qrow * D + hi * HALF) * ES), qf);
 #pragma unroll
   for (int c = 0; c < HALF; ++c) qf[c] *= scale_log2;
 
@@ -136,11 +109,11 @@ fa_f32_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict
     float v[16][NDB];
   };
   auto load_tile = [&](Tile& tl, int j0) {
-    load_row32<T>(k_rs, (uint32_t)(((j0 + lq) * D + hi * HALF) * ES), tl.k);
+    load_row32(k_rs, (uint32_t)(((j0 + lq) * D + hi * HALF) * ES), tl.k);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = j0 + 8 * (r / 4) + 4 * hi + (r % 4);
-      load_pair<T>(v_rs, (uint32_t)((key * D + 2 * lq) * ES), tl.v[r][0], tl.v[r][1]);   // dims 2 lq, 2 lq + 1
+      load_pair(v_rs, (uint32_t)((key * D + 2 * lq) * ES), tl.v[r][0], tl.v[r][1]);   // dims 2 lq, 2 lq + 1
     }
   };
 
@@ -222,18 +195,14 @@ fa_f32_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict
   const float inv = 1.f / l_all;
   // Wave w finalises the (db, g4) groups w, w + KS, ... of its lanes' rows (4 dims each).
   if (qrow < N) {
-    OutT* orow = O + base + (size_t)qrow * D;
+    float* orow = O + base + (size_t)qrow * D;
     for (int grp = wave; grp < NDB * 4; grp += KS) {
       const int db = grp / 4, g4 = grp % 4;
       const int dim = db * 32 + 8 * g4 + 4 * hi;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < KS; ++w) acc += sc[w] * *reinterpret_cast<const f32x4*>(red_o + (w * 32 + lq) * L::LDO + dim);
-      typedef OutT OutV4 __attribute__((ext_vector_type(4)));
-      OutV4 out;
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) out[rr] = from_f32<OutT>(acc[rr] * inv);
-      *reinterpret_cast<OutV4*>(orow + dim) = out;
+      *reinterpret_cast<f32x4*>(orow + dim) = acc * inv;
     }
   }
 }

@@ -133,29 +133,46 @@ template <int CR> __device__ __forceinline__ int v_swz(int row) { return CR == 1
 // form 193 (held to 168 it spills 10 VGPRs and runs 4-26 % faster: B*H x N = 256 x 512 404 -> 422,
 // 128 x 1024 516 -> 584, 128 x 2048 641 -> 794, 64 x 4096 692 -> 873, 16 x 8192 713 -> 887
 // TFLOP/s); the fp16 persistent forms with the packed-max check (CHECK) take 169-171 and are held
-// to 168 (1 VGPR spilled; the ragged one 21).
+// to 168 (1 VGPR spilled; the ragged one 21). The two-term forms take 206-256 and are held to two
+// (three spill 52-56 VGPRs in the causal and ragged forms: fp32-out 2x4x4000 335 TFLOP/s against 477).
 #ifndef PA_MFMA_MIN_WAVES
 #define PA_MFMA_MIN_WAVES 0
 #endif
-template <typename T, int D, bool PERSIST, bool RAGGED, bool CAUSAL, bool CHECK>
+template <typename T, int D, bool PERSIST, bool RAGGED, bool CAUSAL, bool CHECK, int TERMS>
 constexpr int mfma_min_waves() {
   return PA_MFMA_MIN_WAVES > 0 ? PA_MFMA_MIN_WAVES
-                               : (PERSIST && D == 64 && (std::is_same<T, bf16>::value || RAGGED || CAUSAL || CHECK)) ? 3 : 1;
+                               : TERMS == 2 ? 2 : (PERSIST && D == 64 && (std::is_same<T, bf16>::value || RAGGED || CAUSAL || CHECK)) ? 3 : 1;
 }
 
+// TERMS == 2 (fp16, the row-max forms; the `fused` entry's fp16 calls, which promise fp32 arithmetic):
+// P is not rounded to fp16 but taken as two fp16 terms, hi = round(P') and lo = round(P' - hi), 22
+// significant bits, and both go through P.V and the row sum. Products of fp16 values are exact in
+// the fp32 accumulator, and so is Q K^T, so the result has fp32 arithmetic's error: against float64,
+// fp32 output, B x H x N = 1x42x128 / 4x16x2048 / 4x4x8192 / causal 4x4x8000 / 2x4x4000 with Q, K x3,
+// the fp32 matrix core's kernel was 3.0e-7 / 5.2e-7 / 8.8e-7 / 3.8e-7 / 1.5e-6 off and this one
+// 1.7e-7 / 3.6e-7 / 6.3e-7 / 2.6e-7 / 6.1e-7 (2-norms). What keeps it there: O's lo products have an
+// accumulator of their own, and l takes one fp32 add per tile (into one accumulator each, the error
+// grew past the fp32 kernel's at N = 2048). Bound: softmax VALU and matrix core about evenly (24
+// MFMAs of 32x32x16 and 8 of 16x16x32 per 64-key tile against ~5 VALU instructions a score), where
+// the fp32 matrix core has 1/16 of the rate. Time, fp32 matrix core -> this: 4x16x4096 2347 -> 469 us
+// (117 -> 586 TFLOP/s), 8x16x1024 315 -> 63 us, causal 4x16x1024 108 -> 23 us, 1x42x128 6.0 -> 5.0.
+// The interleave (8 and 4 VALU instructions per MFMA) is within 2 % for 4-8 and 3-6.
 // CHECK (fp16, two stages, no key split, not the causal form): the lazy rescale is triggered by a
 // check on the computed P' (as the bf16 kernels always do) instead of the row max of S before the
 // exponentials; see the branch below.
 template <typename T, int D, int BM, int BN, int STAGES, typename OutT, int KSPLIT = 1, bool PERSIST = false,
-          bool RAGGED = false, bool CAUSAL = false, bool CHECK = false>
+          bool RAGGED = false, bool CAUSAL = false, bool CHECK = false, int TERMS = 1>
 __global__ void __launch_bounds__(BM / 32 * kWave * KSPLIT)
-__attribute__((amdgpu_waves_per_eu(mfma_min_waves<T, D, PERSIST, RAGGED, CAUSAL, CHECK>())))
+__attribute__((amdgpu_waves_per_eu(mfma_min_waves<T, D, PERSIST, RAGGED, CAUSAL, CHECK, TERMS>())))
 fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
             OutT* __restrict__ O, int N, int num_qblocks, int total_blocks, float scale_log2, int causal,
             int cus_per_xcd, int walk) {
   typedef typename vec8<T>::type V8;
   typedef MfmaLds<D, BN, STAGES> L;
   constexpr float kLazyLog2 = 8.f;       // P stays below 2^kLazyLog2 between rescales
+  // TERMS == 2: P is taken 2^7 larger (its reference m - 7, in numerator and denominator alike), so
+  // P' <= 2^15 < 65504 and its lo term stays a normal fp16 down to P = 2^-10.
+  constexpr float kTermShift = TERMS == 2 ? 7.f : 0.f;
   constexpr int NW = BM / 32;
   constexpr int THREADS = NW * kWave;
   constexpr int QK_STEPS = D / 16;       // MFMA k-steps over the head dim
@@ -165,7 +182,8 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
   constexpr int CR = D / 8;              // 16-byte chunks per K/V row
   constexpr int RB = L::ROW_BYTES;
   constexpr int QK_MFMAS = NKB * QK_STEPS;
-  constexpr int PV_MFMAS = PV_STEPS * NDB;
+  constexpr int PF = PV_STEPS * TERMS;   // P operands of a tile: the hi terms, then (TERMS == 2) the lo terms
+  constexpr int PV_MFMAS = PF * NDB;
   static_assert(D == 64 || D == 128, "head dim");
   static_assert(BM % 32 == 0 && BN % 32 == 0, "tile shape");
   static_assert((BN * CR) % THREADS == 0, "K/V tile must split evenly over the workgroup");
@@ -179,6 +197,8 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
   static_assert(!PERSIST || (KSPLIT == 1 && STAGES == 2), "persistent form: two stages, no key split");
   static_assert(!RAGGED || PERSIST, "RAGGED selects the persistent form whose last key tile is partial");
   static_assert(!CAUSAL || (PERSIST && !RAGGED && BM % (2 * BN) == 0), "CAUSAL selects the persistent causal form");
+  static_assert(TERMS == 1 || (TERMS == 2 && std::is_same<T, f16>::value && STAGES == 2 && !CHECK),
+                "two-term P: the fp16 two-stage forms with the row max");
   static_assert(!CHECK || (std::is_same<T, f16>::value && STAGES == 2 && KSPLIT == 1 && !CAUSAL),
                 "CHECK: the fp16 two-stage forms without key split, not the causal one");
 
@@ -322,8 +342,21 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
     for (int j = 0; j < 8; ++j) ones[j] = from_f32<T>(on ? 1.f : 0.f);
   }
   f32x16 o[NDB];
+  // TERMS == 2: the lo terms' products, summed apart (half the roundings at the size of O, and an
+  // infinite V meets a lo term of either sign without turning O into a NaN) and added at the end.
+  f32x16 o_lo[TERMS == 2 ? NDB : 1];
 #pragma unroll
-  for (int db = 0; db < NDB; ++db) o[db] = f32x16{};
+  for (int db = 0; db < NDB; ++db) {
+    o[db] = f32x16{};
+    if constexpr (TERMS == 2) o_lo[db] = f32x16{};
+  }
+  auto fold_terms = [&]() {
+    if constexpr (TERMS == 2)
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] = __builtin_isfinite(o[db][r]) ? o[db][r] + o_lo[db][r] : o[db][r];
+  };
 
   const int kv_end = causal ? min(N, q0 + BM) : N;
   // (CAUSAL: the block's tile counts, set again for every block of the walk.)
@@ -409,7 +442,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
   };
 
   // P = 2^(S*c - m) rounded to T: the PV operand.
-  auto exponentiate = [&](const f32x16 (&s)[NKB], V8 (&pf)[PV_STEPS]) {
+  auto exponentiate = [&](const f32x16 (&s)[NKB], V8 (&pf)[PF]) {
     const float neg_m = (m_run == -INFINITY) ? 0.f : -m_run;  // fully masked row: P = 0
 #pragma unroll
     for (int b = 0; b < NKB; ++b)
@@ -418,19 +451,30 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
   };
   // l += sum of the rounded P: 16x16x32 MFMAs of the 0/1 operand by P^T (exact products, fp32
   // accumulation).
-  auto row_sum = [&](const V8 (&pf)[PV_STEPS]) {
+  auto row_sum = [&](const V8 (&pf)[PF]) {
+    if constexpr (TERMS == 2) {
+      // A tile's sum first, then one fp32 add to l (instead of 2 PV_STEPS roundings at l's size).
+      f32x4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks_ = 0; ks_ < PV_STEPS; ++ks_) lacc = mfma16x16x32(ones, pf[ks_], lacc);
+      for (int i = 0; i < PF; ++i) t = mfma16x16x32(ones, pf[PF - 1 - i], t);
+      lacc[0] += t[0];
+    } else {
+#pragma unroll
+      for (int ks_ = 0; ks_ < PF; ++ks_) lacc = mfma16x16x32(ones, pf[ks_], lacc);
+    }
   };
 
   auto rescale_o = [&](float alpha) {
-    lacc *= alpha;
+    if constexpr (TERMS == 2) lacc[0] *= alpha; else lacc *= alpha;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) o[db] *= alpha;
+    for (int db = 0; db < NDB; ++db) {
+      o[db] *= alpha;
+      if constexpr (TERMS == 2) o_lo[db] *= alpha;
+    }
   };
 
   // O^T += V^T . P^T for the tile in V stage `vs`.
-  auto pv = [&](const V8 (&pf)[PV_STEPS], const unsigned char* vs) {
+  auto pv = [&](const V8 (&pf)[PF], const unsigned char* vs) {
 #pragma unroll
     for (int ks_ = 0; ks_ < PV_STEPS; ++ks_) {
 #pragma unroll
@@ -440,6 +484,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
         const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0 + 8 * RB));
         const i16x8 a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
         o[db] = mfma32x32x16(__builtin_bit_cast(V8, a), pf[ks_], o[db]);
+        if constexpr (TERMS == 2) o_lo[db] = mfma32x32x16(__builtin_bit_cast(V8, a), pf[PV_STEPS + ks_], o_lo[db]);
       }
     }
   };
@@ -606,7 +651,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
     };
     // `opaque` hides -m_ref behind an empty asm so that the fast path's exponentials are not
     // merged with the generic path's and hoisted out of the MFMA phases.
-    auto exp_range = [&](const f32x16 (&s_)[NKB], V8 (&pf)[PV_STEPS], int lo, int hi, bool opaque) __attribute__((always_inline)) {
+    auto exp_range = [&](const f32x16 (&s_)[NKB], V8 (&pf)[PF], int lo, int hi, bool opaque) __attribute__((always_inline)) {
       float nm = -m_ref;
       if (opaque) asm("" : "+v"(nm));
 #pragma unroll
@@ -640,11 +685,11 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
     // their OR (`or_c`) come from iteration t-1 (for tile 0, from the prologue, after the first
     // tile's exact max).
     f32x16 sa[NKB], sb[NKB];
-    V8 pa[PV_STEPS], pb[PV_STEPS];
+    V8 pa[PF], pb[PF];
     uint32_t or_c = kForce;
     // S(0) and the first half of P'(0) of a block (the arrays are parameters, not captures:
     // capturing them here changes how the compiler allocates the whole kernel).
-    auto first_tile = [&](f32x16 (&s0)[NKB], V8 (&p0)[PV_STEPS]) {
+    auto first_tile = [&](f32x16 (&s0)[NKB], V8 (&p0)[PF]) {
       if (tile_of(0) < wave_tiles) {
         qk(s0, k_stage(even));
         if (!PERSIST && tile_of(0) >= clean_tiles) mask(s0, tile_of(0) * BN);
@@ -670,8 +715,8 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
 
     // `par` is the parity of t as a compile-time constant, so every stage below is a fixed LDS
     // object: K(t+1) in k_stage(!par), V(t) in v_stage(par).
-    auto iteration = [&](auto par, auto wrap, int t, f32x16 (&s)[NKB], f32x16 (&sn)[NKB], V8 (&pf)[PV_STEPS],
-                         V8 (&pn)[PV_STEPS]) {
+    auto iteration = [&](auto par, auto wrap, int t, f32x16 (&s)[NKB], f32x16 (&sn)[NKB], V8 (&pf)[PF],
+                         V8 (&pn)[PF]) {
       constexpr int P = decltype(par)::value;
       // WRAP: the persistent form's last two iterations of a block (t = nit-2, nit-1): loads past
       // the block's last tile fetch the next block's first tiles instead; the last one has no
@@ -782,7 +827,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
           // V operand reads (two per MFMA) run two MFMAs ahead of their use.
           __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4, 0);
 #pragma unroll
-          for (int i = 0; i < PV_MFMAS + PV_STEPS; ++i) {
+          for (int i = 0; i < PV_MFMAS + PF; ++i) {
             __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
             __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 0);
             __builtin_amdgcn_sched_group_barrier(kSchedValu, VB, 0);
@@ -871,6 +916,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
           iteration(even, with_wrap, nit - 2, sa, sb, pa, pb);
           iteration(odd, with_wrap, nit - 1, sb, sa, pb, pa);
         }
+        if constexpr (TERMS == 2) fold_terms();
         store_block();
         if (!has_next) break;
         ++step;
@@ -890,7 +936,10 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
         k_rs = make_rsrc(K + base, head_bytes);
         v_rs = make_rsrc(V + base, head_bytes);
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) o[db] = f32x16{};
+        for (int db = 0; db < NDB; ++db) {
+          o[db] = f32x16{};
+          if constexpr (TERMS == 2) o_lo[db] = f32x16{};
+        }
         lacc = f32x4{0.f, 0.f, 0.f, 0.f};
         m_ref = -3.0e38f;
         // K(0), K(1), V(0) and Q landed with the last iteration's wait; V(1) comes with
@@ -909,7 +958,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
     // Two score buffers swap roles every iteration (the loop is unrolled by two so the swap
     // costs no register moves).
     f32x16 sa[NKB], sb[NKB];
-    V8 pa[PV_STEPS], pb[PV_STEPS];
+    V8 pa[PF], pb[PF];
     bool rescale = false;
     float alpha = 1.f;
     // The first QB P operand registers of tile t+1 are made in phase B of iteration t, right after
@@ -919,18 +968,22 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
     // 64 x 64 one runs 2-7 % faster with the split; that tile (6 %) and d = 128 (1 %, where 16
     // MFMAs per phase already carry the exponentials) run faster with all of P(t) in phase A.
     constexpr int QB = (D == 128 || (BM == 64 && BN == 64)) ? 0 : PV_STEPS / 2;
-    auto exp_part = [&](const f32x16 (&s_)[NKB], V8 (&p_)[PV_STEPS], int lo, int hi, bool opaque) __attribute__((always_inline)) {
-      float nm = (m_run == -INFINITY) ? 0.f : -m_run;  // fully masked row: P = 0
+    auto exp_part = [&](const f32x16 (&s_)[NKB], V8 (&p_)[PF], int lo, int hi, bool opaque) __attribute__((always_inline)) {
+      float nm = (m_run == -INFINITY) ? 0.f : kTermShift - m_run;  // fully masked row: P = 0
       if (opaque) asm("" : "+v"(nm));
 #pragma unroll
       for (int i = 0; i < PV_STEPS; ++i)
         if (i >= lo && i < hi)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) p_[i][j] = from_f32<T>(exp2_fast(fmaf(s_[i / 2][8 * (i % 2) + j], scale_log2, nm)));
+          for (int j = 0; j < 8; ++j) {
+            const float x = exp2_fast(fmaf(s_[i / 2][8 * (i % 2) + j], scale_log2, nm));
+            p_[i][j] = from_f32<T>(x);
+            if constexpr (TERMS == 2) p_[PV_STEPS + i][j] = from_f32<T>(fmaf(-1.f, to_f32(p_[i][j]), x));
+          }
     };
     // S(0), its row max and the first QB P registers of a block (arrays as parameters, not
     // captures, as on the bf16 path).
-    auto first_tile = [&](f32x16 (&s0)[NKB], V8 (&p0)[PV_STEPS]) {
+    auto first_tile = [&](f32x16 (&s0)[NKB], V8 (&p0)[PF]) {
       if (tile_of(0) < wave_tiles) {
         qk(s0, k_stage(even));
         if (!PERSIST && tile_of(0) >= clean_tiles) mask(s0, tile_of(0) * BN);
@@ -952,8 +1005,8 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
 
     // `par` is the parity of t as a compile-time constant, so every stage below is a fixed LDS
     // object: K(t+1) in k_stage(!par), V(t) in v_stage(par).
-    auto iteration = [&](auto par, auto wrap, int t, f32x16 (&s)[NKB], f32x16 (&sn)[NKB], V8 (&pf)[PV_STEPS],
-                         V8 (&pn)[PV_STEPS]) {
+    auto iteration = [&](auto par, auto wrap, int t, f32x16 (&s)[NKB], f32x16 (&sn)[NKB], V8 (&pf)[PF],
+                         V8 (&pn)[PF]) {
       constexpr int P = decltype(par)::value;
       // WRAP: the persistent form's last two iterations of a block; the loads past the block's
       // last tile fetch the next block's K(0), K(1), V(0) and Q (as on the bf16 path). DIAG: as
@@ -988,8 +1041,8 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
             constexpr bool RS = decltype(with_rescale)::value;
             // (the fused_tc d = 64 tile measured fastest at 4 and, in phase B, 8: C3 +0.5 %,
             // C5 +0.6 % over the per-phase totals 5 and 11, within 1 % for 4-6 and 4-11)
-            constexpr int VA = (D == 64 && BM == 128 && BN == 64 && !RS)
-                                   ? 4 : ((PV_STEPS - QB) * 20 + (RS ? NDB * 16 + 2 : 0) + QK_MFMAS - 1) / QK_MFMAS;
+            constexpr int VA = TERMS == 2 ? 8 : (D == 64 && BM == 128 && BN == 64 && !RS)
+                                   ? 4 : ((PV_STEPS - QB) * 20 + (RS ? NDB * 16 * TERMS + 2 : 0) + QK_MFMAS - 1) / QK_MFMAS;
             // Phase A at wave priority 2, as on the bf16 path (causal fp16 d = 64 4x16x1024 +2.1-3.1 %,
             // 1x16x2048 +1.0-1.2 %); not in the key split, which lost 8 % with it (C2, 1x4x8192).
             if constexpr (KSPLIT == 1) __builtin_amdgcn_s_setprio(2);
@@ -1013,7 +1066,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
             if (t + 2 == wave_tiles) mask_diag(sn, (t + 1) * BN);
           }
           // Phase B: PV(t) MFMAs with the row sum of P(t) and the row max of S(t+1).
-          constexpr int VB = (D == 64 && BM == 128 && BN == 64) ? 8 : (NKB * 8 + 10 + QB * 20 + PV_MFMAS - 1) / PV_MFMAS;
+          constexpr int VB = TERMS == 2 ? 4 : (D == 64 && BM == 128 && BN == 64) ? 8 : (NKB * 8 + 10 + QB * 20 + PV_MFMAS - 1) / PV_MFMAS;
           pv(pf, vc);
           row_sum(pf);
           alpha = update_max(sn, rescale);
@@ -1021,7 +1074,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
           // V operand reads (two per MFMA) run two MFMAs ahead of their use.
           __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 4, 0);
 #pragma unroll
-          for (int i = 0; i < PV_MFMAS + PV_STEPS; ++i) {
+          for (int i = 0; i < PV_MFMAS + PF; ++i) {
             __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
             __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 0);
             __builtin_amdgcn_sched_group_barrier(kSchedValu, VB, 0);
@@ -1032,7 +1085,10 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
           // (across the barrier), leaving that phase A 32 exponentials against 8 MFMAs and the
           // phase B before it none (C3, C5 +0.8 %, 8 fewer VGPRs).
 #pragma unroll
-          for (int i = 0; i < QB; ++i) asm volatile("" : "+v"(pn[i]));
+          for (int i = 0; i < QB; ++i) {
+            asm volatile("" : "+v"(pn[i]));
+            if constexpr (TERMS == 2) asm volatile("" : "+v"(pn[PV_STEPS + i]));
+          }
         } else {
           // Generic path: the next tile is masked or absent.
           const bool ahead = tile_of(t + 1) < wave_tiles;
@@ -1089,6 +1145,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
           iteration(even, with_wrap, nit - 2, sa, sb, pa, pb);
           iteration(odd, with_wrap, nit - 1, sb, sa, pb, pa);
         }
+        if constexpr (TERMS == 2) fold_terms();
         store_block();
         if (!has_next) break;
         ++step;
@@ -1105,7 +1162,10 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
         k_rs = make_rsrc(K + base, head_bytes);
         v_rs = make_rsrc(V + base, head_bytes);
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) o[db] = f32x16{};
+        for (int db = 0; db < NDB; ++db) {
+          o[db] = f32x16{};
+          if constexpr (TERMS == 2) o_lo[db] = f32x16{};
+        }
         lacc = f32x4{0.f, 0.f, 0.f, 0.f};
         m_run = -INFINITY;
         rescale = false;
@@ -1125,7 +1185,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
       __syncthreads();
       if (t < wave_tiles) {
         f32x16 s[NKB];
-        V8 pf[PV_STEPS];
+        V8 pf[PF];
         bool rescale;
         qk(s, k_stage(even));
         if (t >= clean_tiles) mask(s, j0);
@@ -1137,6 +1197,8 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
       }
     }
   }
+
+  if constexpr (!PERSIST && TERMS == 2) fold_terms();
 
   // ---- Key groups: group 1 hands (m, l, O) to the lane of group 0 that holds the same query and
   // dims, through the (now free) K/V stages; group 0 merges them with the online-softmax rule

@@ -127,14 +127,14 @@ int persistent_grid(long long total_blocks, int wgs_per_cu) {
 // Workgroups of an fa_mfma_fwd instantiation that fit on one CU of the current device (queried
 // once per device), 0 if unknown.
 template <typename T, int D, int BM, int BN, int ST, typename OutT, int KS, bool PERSIST, bool RAGGED, bool CAUSAL,
-          bool CHECK = false>
+          bool CHECK = false, int TERMS = 1>
 int wgs_per_cu() {
   static std::atomic<int> cache[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
   int n = cache[dev].load(std::memory_order_relaxed);
   if (n == 0) {
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, PERSIST, RAGGED, CAUSAL, CHECK>,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, PERSIST, RAGGED, CAUSAL, CHECK, TERMS>,
                                                      BM / 32 * pa::kWave * KS, 0) != hipSuccess || n <= 0)
       return 0;
     cache[dev].store(n, std::memory_order_relaxed);
@@ -154,13 +154,13 @@ struct PersistentPlan {
   int grid = 0;      // workgroups of the persistent launch, 0 for one workgroup per query block
   int walk = 0;      // causal walk: 0 per-XCD lists head by head, 1 per-XCD lists by length, 2 one list
 };
-template <typename T, int D, int BM, int BN, int ST, typename OutT, int KS>
+template <typename T, int D, int BM, int BN, int ST, typename OutT, int KS, int TERMS = 1>
 PersistentPlan persistent_grid_for(int64_t n, int64_t bh, int causal) {
   static_assert(ST == 2 && KS == 1, "persistent forms: two stages, no key split");
   if (!persistent_launch(n, BN, causal)) return {};
   const long long total = (n + BM - 1) / BM * bh;
   if (causal) {
-    const int wpc = wgs_per_cu<T, D, BM, BN, ST, OutT, KS, true, false, true>();
+    const int wpc = wgs_per_cu<T, D, BM, BN, ST, OutT, KS, true, false, true, false, TERMS>();
     const int cus = device_cus() / pa::kNumXcd;
     // Per-XCD lists (each XCD owning whole heads) need B*H a multiple of 8, or else at most 25 %
     // more heads on the busiest XCD than the mean and a block for every workgroup on every XCD
@@ -176,10 +176,10 @@ PersistentPlan persistent_grid_for(int64_t n, int64_t bh, int causal) {
     if (grid <= 0) return {};
     return {grid, pa::causal_walk(n, bh, BM, BN, grid / pa::kNumXcd, cus, D == 64, per_xcd)};
   }
-  constexpr bool kCheck = std::is_same<T, pa::f16>::value;   // the fp16 non-causal forms' packed-max check
-  const int clean = wgs_per_cu<T, D, BM, BN, ST, OutT, KS, true, false, false, kCheck>();
+  constexpr bool kCheck = TERMS == 1 && std::is_same<T, pa::f16>::value;   // the fp16 non-causal forms' packed-max check
+  const int clean = wgs_per_cu<T, D, BM, BN, ST, OutT, KS, true, false, false, kCheck, TERMS>();
   if (n % (2 * BN) == 0) return {persistent_grid(total, clean), 0};
-  const int ragged = wgs_per_cu<T, D, BM, BN, ST, OutT, KS, true, true, false, kCheck>();
+  const int ragged = wgs_per_cu<T, D, BM, BN, ST, OutT, KS, true, true, false, kCheck, TERMS>();
   return ragged >= clean ? PersistentPlan{persistent_grid(total, ragged), 0} : PersistentPlan{};
 }
 
@@ -193,24 +193,24 @@ PersistentPlan persistent_grid_for(int64_t n, int64_t bh, int causal) {
 // 748 -> 744; d = 128 4x32x4096 1080 -> 1152. Per block: d = 128 4x32x4096 1048 -> 1100, 1x32x1030
 // 487 -> 524; d = 64 it lost (2 waves per SIMD, 194 VGPRs: C3 716 -> 696, 8x16x1025 602 -> 554;
 // held to 3 with 16 VGPRs spilled: 437), and on causal d = 64 rows 9 % at 8x16x1024.
-template <typename T, int D, int BM, int BN, int ST, typename OutT, int KS = 1, bool TC = false>
+template <typename T, int D, int BM, int BN, int ST, typename OutT, int KS = 1, bool TC = false, int TERMS = 1>
 hipError_t launch_mfma(const void* q, const void* k, const void* v, void* o, int bh, int n, int causal,
                        hipStream_t stream) {
   const int qblocks = (n + BM - 1) / BM;
   const long long total = (long long)qblocks * bh;
   if (total > INT_MAX) return hipErrorInvalidConfiguration;
-  constexpr bool kCheck = TC && ST == 2 && KS == 1 && std::is_same<T, pa::f16>::value;
+  constexpr bool kCheck = TC && TERMS == 1 && ST == 2 && KS == 1 && std::is_same<T, pa::f16>::value;
   constexpr bool kCheckPerBlock = kCheck && D == 128;
   if constexpr (TC && ST == 2 && KS == 1) {
     {
-      const PersistentPlan plan = persistent_grid_for<T, D, BM, BN, ST, OutT, KS>(n, bh, causal);
+      const PersistentPlan plan = persistent_grid_for<T, D, BM, BN, ST, OutT, KS, TERMS>(n, bh, causal);
       if (plan.grid > 0) {
         // Non-causal with N a multiple of 2 * BN: an even number of full tiles. Otherwise (an
         // even tile count whose last tile is partial, or an odd count of full tiles, padded with
         // an empty one) the RAGGED form, whose wrap copies mask the keys past N.
-        auto kernel = causal ? pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, true, false, true>
-                      : n % (2 * BN) == 0 ? pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, true, false, false, kCheck>
-                                          : pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, true, true, false, kCheck>;
+        auto kernel = causal ? pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, true, false, true, false, TERMS>
+                      : n % (2 * BN) == 0 ? pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, true, false, false, kCheck, TERMS>
+                                          : pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, true, true, false, kCheck, TERMS>;
         hipLaunchKernelGGL(kernel, dim3((unsigned)plan.grid), dim3(BM / 32 * pa::kWave * KS), 0, stream,
                            static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
                            static_cast<OutT*>(o), n, qblocks, (int)total, scale_log2_for(D), causal,
@@ -219,8 +219,8 @@ hipError_t launch_mfma(const void* q, const void* k, const void* v, void* o, int
       }
     }
   }
-  auto kernel = kCheckPerBlock && !causal ? pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, false, false, false, kCheckPerBlock>
-                                          : pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS>;
+  auto kernel = kCheckPerBlock && !causal ? pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, false, false, false, kCheckPerBlock, TERMS>
+                                          : pa::fa_mfma_fwd<T, D, BM, BN, ST, OutT, KS, false, false, false, false, TERMS>;
   hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(BM / 32 * pa::kWave * KS), 0, stream,
                      static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
                      static_cast<OutT*>(o), n, qblocks, (int)total, scale_log2_for(D), causal, 0, 0);
@@ -358,20 +358,29 @@ const MfmaEntry* find_tuned(int dtype, int out_dtype, int64_t d, int br, int bc,
   return nullptr;
 }
 
-// ------------------------------------------------------------------ fused fp32 arithmetic
-// 32 query rows per workgroup, keys split over kF32KS waves (merged through LDS at the end).
+// ------------------------------------------------------------------ fused, fp32 arithmetic
+// fp32 inputs: 32 query rows per workgroup, keys split over kF32KS waves (merged through LDS at the end).
 constexpr int kF32KS = 4;
 
-template <typename T, typename OutT>
 hipError_t launch_f32(const void* q, const void* k, const void* v, void* o, int bh, int n, int causal,
                       hipStream_t stream) {
   const int qblocks = (n + 31) / 32;
   const long long total = (long long)qblocks * bh;
   if (total > INT_MAX) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((pa::fa_f32_fwd<T, 64, kF32KS, OutT>), dim3((unsigned)total), dim3(kF32KS * pa::kWave),
-                     0, stream, static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
-                     static_cast<OutT*>(o), n, qblocks, (int)total, scale_log2_for(64), causal);
+  hipLaunchKernelGGL((pa::fa_f32_fwd<64, kF32KS>), dim3((unsigned)total), dim3(kF32KS * pa::kWave),
+                     0, stream, static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
+                     static_cast<float*>(o), n, qblocks, (int)total, scale_log2_for(64), causal);
   return hipGetLastError();
+}
+
+// fp16 inputs: the fp16 matrix core with P in two terms, in fused_tc's launch forms (persistent, or
+// the key split on the grids use_key_split names; the same rule, since both have the same blocks).
+template <typename OutT>
+hipError_t launch_f16_terms(const void* q, const void* k, const void* v, void* o, int bh, int n, int causal,
+                            hipStream_t stream) {
+  return use_key_split(64, n, bh, causal)
+             ? launch_mfma<pa::f16, 64, 64, 64, 2, OutT, 2, false, 2>(q, k, v, o, bh, n, causal, stream)
+             : launch_mfma<pa::f16, 64, 128, 64, 2, OutT, 1, true, 2>(q, k, v, o, bh, n, causal, stream);
 }
 
 // ------------------------------------------------------------------ unfused
@@ -570,11 +579,11 @@ int pa_fused_fwd(const void* q, const void* k, const void* v, void* o, int dtype
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
   if (dtype == PA_DTYPE_F32 && out_dtype == PA_DTYPE_F32)
-    e = launch_f32<float, float>(q, k, v, o, (int)bh, (int)n, causal, st);
+    e = launch_f32(q, k, v, o, (int)bh, (int)n, causal, st);
   else if (dtype == PA_DTYPE_F16 && out_dtype == PA_DTYPE_F16)
-    e = launch_f32<pa::f16, pa::f16>(q, k, v, o, (int)bh, (int)n, causal, st);
+    e = launch_f16_terms<pa::f16>(q, k, v, o, (int)bh, (int)n, causal, st);
   else if (dtype == PA_DTYPE_F16 && out_dtype == PA_DTYPE_F32)
-    e = launch_f32<pa::f16, float>(q, k, v, o, (int)bh, (int)n, causal, st);
+    e = launch_f16_terms<float>(q, k, v, o, (int)bh, (int)n, causal, st);
   else
     return fail(PA_ERR_UNSUPPORTED, "%s: only float32 and float16 are supported", name);
   return hip_status(e, name);

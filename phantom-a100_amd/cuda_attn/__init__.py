@@ -10,7 +10,7 @@ through its C ABI (include/phantom_attn.h); there is no CPU or PyTorch fallback.
 
     naive        3 kernels, fp32 N x N scores in a workspace        any d, fp32/fp16
     tiled        LDS-tiled scores / P.V, one wave per softmax row     any d, fp32/fp16
-    fused        fused online softmax, fp32 arithmetic (fp32 MFMA)    d=64, fp32/fp16
+    fused        fused online softmax, fp32 arithmetic on MFMA        d=64, fp32/fp16
     fused_tuned  fp16 MFMA fused kernel at a chosen (br, bc) tile and 1 or 2 LDS stages
     fused_tc     fp16/bf16 MFMA fused kernel                          d=64 or 128
 

@@ -432,6 +432,41 @@ def test_fused_tc_matches_rounded_p_model(path):
     assert err <= tol, f"vs the kernel model {err:.3e} > {tol:.1e} (reference algorithm vs float64: {e_ref:.2e})"
 
 
+# fused with fp16 inputs: fp32 arithmetic on the fp16 matrix core (P in two fp16 terms).
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("bh,n", [(3, 1), (3, 31), (3, 64), (42, 65), (42, 128), (42, 129), (5, 191), (300, 192),
+                                  (300, 200), (300, 256), (300, 320), (3, 2049), (140, 1000)])
+def test_fused_fp16_inputs_keep_fp32_arithmetic(bh, n, causal):
+    """fp32 output of fp16 inputs against float64, at the edges of the 64-key tiles, of the key split
+    and of the persistent forms (even, odd and partial last tiles), held to the fp32 bar: products of
+    fp16 values are exact in fp32, P carries 22 significant bits (2^-22 of it, 2.4e-7) and |V| < 6."""
+    q, k, v = gpu_qkv(1, bh, n, 64, torch.float16, seed=n)
+    ref = f64_reference_gpu(q, k, v, causal)
+    out = cuda_attn.fused(q, k, v, causal, out_dtype=torch.float32)
+    assert (out.double() - ref).abs().max().item() <= F32_BAR
+    prev = _native.set_persistent(False)   # one workgroup per query block: the same arithmetic
+    try:
+        assert torch.equal(cuda_attn.fused(q, k, v, causal, out_dtype=torch.float32), out)
+    finally:
+        _native.set_persistent(prev)
+    half = cuda_attn.fused(q, k, v, causal)
+    assert torch.equal(half, out.half())
+
+
+def test_fused_fp16_infinite_value_stays_infinite():
+    """An infinite element of V gives an infinite (not NaN) output in its dim where its weight is not
+    tiny, as a product with an fp32 weight does; the other dims are not touched."""
+    q, k, v = gpu_qkv(1, 2, 300, 64, torch.float16, seed=7)
+    want = cuda_attn.fused(q, k, v, out_dtype=torch.float32)
+    v[0, 0, 17, 5] = float("inf")
+    v[0, 1, 200, 9] = -float("inf")
+    out = cuda_attn.fused(q, k, v, out_dtype=torch.float32)
+    assert (out[0, 0, :, 5] == float("inf")).all() and (out[0, 1, :, 9] == -float("inf")).all()
+    keep = torch.ones_like(out, dtype=torch.bool)
+    keep[0, 0, :, 5] = keep[0, 1, :, 9] = False
+    assert torch.equal(out[keep], want[keep])
+
+
 # ---------------------------------------------------------------- 3. BASELINE configs, full size
 CONFIG_TOL = {"C1": 1e-5, "C2": 2e-3, "C3": 2e-3, "C4": 2e-3, "C5": 2e-3}
 
