@@ -20,6 +20,7 @@
 
 #include "phantom_attn.h"
 #include "kernels/fa_f32.hpp"
+#include "kernels/fa_f32x3.hpp"
 #include "kernels/fa_mfma.hpp"
 #include "kernels/unfused.hpp"
 #include "launch_model.hpp"
@@ -359,11 +360,41 @@ const MfmaEntry* find_tuned(int dtype, int out_dtype, int64_t d, int br, int bc,
 }
 
 // ------------------------------------------------------------------ fused, fp32 arithmetic
-// fp32 inputs: 32 query rows per workgroup, keys split over kF32KS waves (merged through LDS at the end).
+// fp32 inputs, three kernels. fa_f32_fwd (fp32 matrix core): 32 query rows per workgroup, keys split
+// over kF32KS waves. fa_f32x3_fwd (bf16 matrix core, three-term operands): 128 query rows per
+// workgroup, in one key group of 4 waves or two of them.
 constexpr int kF32KS = 4;
+// The bf16 terms have 2.7x the fp32 matrix core's rate but a quarter of its workgroups (four waves
+// share a staged tile; with their own tiles the splitting costs what the rate gains), so they are
+// taken where the 128-query blocks outnumber half the CUs (short rows: 160, the staging is a larger
+// part of them) and a row has more than one 32-key tile. Measured, fa_f32_fwd -> fa_f32x3_fwd in us:
+// 64 heads x 256 (128 blocks) 15.2 -> 15.7, 16x1000 (128) 44.7 -> 43.1, causal 3x5000 (120) 153 ->
+// 181, 150x96 9.0 -> 9.6; above the line 96x256 (192) 22.8 -> 16.2, 9x2048 (144) 118 -> 79, causal
+// 5x4096 (160) 166 -> 150, 200x64 8.3 -> 7.8, 400x33 14.3 -> 10.5; rows of one tile lose at any
+// count (1000x32 10.5 -> 13.0).
+bool use_bf16_terms(int64_t n, int64_t blocks) { return n > 32 && blocks > (n <= 128 ? 160 : 128); }
+// Two key groups (8 waves, one workgroup per CU) where one group would leave the CUs a workgroup of
+// 4 waves or less to end on: up to one block per CU, and up to two for rows of 1024 keys or more.
+// One group -> two, us: 96x256 (192) 18.5 -> 16.2, 64x512 (256) 32.7 -> 28.7, causal 7x4096 (224)
+// 216 -> 150, 24x2048 (384) 176 -> 168, causal 40x1024 (320) 60.6 -> 45.9, causal 64x1024 (512)
+// 67 -> 62, 16x4096 (512) 378 -> 360; beyond: causal 128x1024 (1024) 112 -> 123, 100x512 (400) 50.3 ->
+// 51.8, 324x128 (324) 17.9 -> 22.5.
+bool use_f32x3_key_groups(int64_t n, int64_t blocks) {
+  return (n > 128 && blocks <= kCUs) || (n >= 1024 && blocks <= 2 * kCUs);
+}
 
 hipError_t launch_f32(const void* q, const void* k, const void* v, void* o, int bh, int n, int causal,
                       hipStream_t stream) {
+  const long long blocks = (long long)((n + 127) / 128) * bh;
+  if (blocks > INT_MAX) return hipErrorInvalidConfiguration;
+  if (use_bf16_terms(n, blocks)) {
+    const bool groups = use_f32x3_key_groups(n, blocks);
+    auto kernel = groups ? pa::fa_f32x3_fwd<64, 4, 2> : pa::fa_f32x3_fwd<64, 4, 1>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(4 * (groups ? 2 : 1) * pa::kWave), 0, stream,
+                       static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
+                       static_cast<float*>(o), n, (n + 127) / 128, (int)blocks, scale_log2_for(64), causal);
+    return hipGetLastError();
+  }
   const int qblocks = (n + 31) / 32;
   const long long total = (long long)qblocks * bh;
   if (total > INT_MAX) return hipErrorInvalidConfiguration;

@@ -467,6 +467,44 @@ def test_fused_fp16_infinite_value_stays_infinite():
     assert torch.equal(out[keep], want[keep])
 
 
+# fused with fp32 inputs: the fp32 matrix core on small grids, three bf16 terms per operand on larger
+# ones (one or two key groups).
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("bh,n", [(128, 128), (161, 33), (161, 64), (161, 65), (162, 128), (129, 129), (300, 96),
+                                  (260, 160), (64, 257), (70, 255), (17, 1000), (33, 1024), (65, 1023), (9, 2049)])
+def test_fused_fp32_forms(bh, n, causal):
+    """Both kernels and both key-group forms against float64 at the fp32 bar, at the edges of the 32-key
+    tiles (odd and even counts, partial last tiles) and of the dispatch."""
+    q, k, v = gpu_qkv(1, bh, n, 64, torch.float32, seed=n + bh)
+    ref = f64_reference_gpu(q, k, v, causal)
+    out = cuda_attn.fused(q, k, v, causal)
+    assert (out.double() - ref).abs().max().item() <= F32_BAR
+
+
+@pytest.mark.parametrize("bh,n", [(3, 300), (130, 300), (300, 300)])
+def test_fused_fp32_range(bh, n):
+    """Values that no bf16 holds, and infinities, in each of the kernels: finite weights times values
+    up to the largest float (within 2^-20 of them: an exponent argument below 16 is rounded at 2^-21,
+    its scores and 2^x add about as much), an infinite value infinite in
+    its dim alone, and a key whose score is -inf left out."""
+    q, k, v = gpu_qkv(1, bh, n, 64, torch.float32, seed=11)
+    v[0, 0, 7] = 3.4028234e38
+    v[0, 1, 9, 3] = float("inf")
+    q[0, 2, :, 0] = q[0, 2, :, 0].abs() + 0.1
+    k[0, 2, 5, 0] = -float("inf")
+    out = cuda_attn.fused(q, k, v)
+    head = slice(0, 1)
+    ref = f64_reference_gpu(q[:, head], k[:, head], v[:, head])
+    assert ((out[:, head].double() - ref).abs() <= 2.0 ** -20 * ref.abs()).all()
+    want = cuda_attn.fused(q, k, torch.where(v.isinf(), torch.zeros_like(v), v))
+    assert (out[0, 1, :, 3] == float("inf")).all()
+    keep = torch.arange(64, device="cuda") != 3
+    assert torch.equal(out[0, 1][:, keep], want[0, 1][:, keep])
+    rest = torch.arange(n, device="cuda") != 5
+    s = (q[0, 2].double() @ k[0, 2][rest].double().t()) / 8.0
+    assert (out[0, 2].double() - torch.softmax(s, -1) @ v[0, 2][rest].double()).abs().max().item() <= F32_BAR
+
+
 # ---------------------------------------------------------------- 3. BASELINE configs, full size
 CONFIG_TOL = {"C1": 1e-5, "C2": 2e-3, "C3": 2e-3, "C4": 2e-3, "C5": 2e-3}
 
