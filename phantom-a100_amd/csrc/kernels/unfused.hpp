@@ -4,7 +4,7 @@
 // any head dim d >= 1 is accepted, fp32 or fp16 storage, fp32 arithmetic.
 //
 //   naive (/root/reference/csrc/kernels/naive.cuh:10-64): the same three passes (scores, softmax
-//         by row max / sum / normalise, P.V) as plain loops, one wave per row of each product.
+//         by row max / sum / normalise, P.V) as plain loops, a wave taking a few rows of each product.
 //   tiled (/root/reference/csrc/kernels/tiled.cuh:16-117): both products on the matrix core
 //         for fp16 inputs (scores at d a multiple of 16, P.V at d = 64 / 128) and for fp32 inputs
 //         at d = 64 / 128 (tiled_*_mfma, tiled_*_mfma_f32); otherwise 64x64 output tiles with 4x4
@@ -22,54 +22,72 @@ namespace pa {
 
 // ------------------------------------------------------------------------------------ naive
 // The reference's three unfused passes, each a plain loop per lane, laid out by waves: every
-// workgroup is 4 waves, and a wave owns one row of the product it writes (64 keys of a score row,
-// a whole softmax row, 64 head dims of an output row), so the operand that row shares (the query
-// row, the P row) is the same address in every lane, and the per-lane operand (a K row, a V
-// column) is a different one. Grids are flattened into x: N rows times column blocks.
+// workgroup is 4 waves, and a wave owns R rows of the product it writes (64 keys of the score rows,
+// 64 head dims of the output rows; a whole softmax row), so the operand that the rows bring (query
+// rows, P rows) is the same address in every lane, and the per-lane operand (a K row, a V column)
+// serves R rows. One row per wave spent an L1 access on every FMA (a lane's K row piece, a V element);
+// with the rows' operands in scalar registers, R FMAs share it, and what is left is the latency of
+// the loads, issued 16 elements at a time: fp32 2x8x333 d = 80 300 -> 56 us, fp32 8x16x1024 d = 128
+// 19.8 -> 2.3 ms, fp16 324x128 d = 64 223 -> 74 us, fp32 42x128 53 -> 23 us, same bits. Grids are
+// flattened into x: row groups times column blocks.
 
-// S[h][i][j0 + lane] for the wave's query row i and 64 keys from j0; keys after i are -inf when
-// causal. PIECES (rows of whole 16-byte pieces, 16-byte aligned): each lane reads its K row, and
-// the wave its Q row, a 16-byte piece per load instead of an element per load (one load then
-// touches the wave's 64 K rows once per piece, not once per element); the products are summed in
-// the same order either way.
-template <typename T, bool PIECES>
+// S[h][i][j0 + lane] for the wave's R query rows i and 64 keys from j0; keys after i are -inf when
+// causal. A lane's K row element serves the R rows, whose Q elements are the same address in every
+// lane (scalar loads; a row past N reads row N - 1 and is not stored). PIECES (rows of whole 16-byte
+// pieces, 16-byte aligned): K rows are read a 16-byte piece per load instead of an element (one load
+// then touches the wave's 64 K rows once per piece, not once per element); a score's products are
+// summed in dim order either way.
+template <typename T, bool PIECES, int R>
 __global__ void __launch_bounds__(256)
 naive_scores(const T* __restrict__ Q, const T* __restrict__ K, float* __restrict__ S, int N, int d,
              float scale, int causal, int key_blocks) {
-  const int unit = (int)blockIdx.x * 4 + (int)threadIdx.x / kWave;   // (query row, 64-key block)
-  const int i = unit / key_blocks;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int unit = (int)blockIdx.x * 4 + wave;   // (R query rows, 64-key block)
+  const int i0 = unit / key_blocks * R;
   const int j = (unit % key_blocks) * kWave + (int)threadIdx.x % kWave;
-  if (i >= N || j >= N) return;
+  if (i0 >= N || j >= N) return;
   const size_t head = (size_t)blockIdx.y * N;
-  float* srow = S + (head + i) * N;
-  if (causal && j > i) {   // masked: the product is not needed
-    srow[j] = -INFINITY;
-    return;
+  const T* q[R];
+  float dot[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    q[r] = Q + (head + min(i0 + r, N - 1)) * d;
+    dot[r] = 0.f;
   }
-  const T* qi = Q + (head + i) * d;
-  const T* kj = K + (head + j) * d;
-  float dot = 0.f;
-  if constexpr (PIECES) {
-    constexpr int E = 16 / (int)sizeof(T);   // elements per piece
-    for (int c = 0; c < d; c += E) {
-      // (the loaded vector is bit-cast as a whole before its elements are taken)
-      const u32x4 qw = *reinterpret_cast<const u32x4*>(qi + c);
-      const u32x4 kw = *reinterpret_cast<const u32x4*>(kj + c);
-      if constexpr (sizeof(T) == 4) {
-        const f32x4 qv = __builtin_bit_cast(f32x4, qw), kv = __builtin_bit_cast(f32x4, kw);
+  if (!(causal && j > i0 + R - 1)) {   // (masked for every row: the products are not needed)
+    const T* kj = K + (head + j) * d;
+    if constexpr (PIECES) {
+      constexpr int E = 16 / (int)sizeof(T);   // elements per piece
+      constexpr int U = 16 / E;                // pieces per step: their loads are issued together
+      typedef T VecE __attribute__((ext_vector_type(E)));
+      int c = 0;
+      for (; c + 16 <= d; c += 16) {
+        VecE kv[U];
 #pragma unroll
-        for (int e = 0; e < E; ++e) dot = fmaf(qv[e], kv[e], dot);
-      } else {
-        const typename vec8<T>::type qv = __builtin_bit_cast(typename vec8<T>::type, qw);
-        const typename vec8<T>::type kv = __builtin_bit_cast(typename vec8<T>::type, kw);
+        for (int u = 0; u < U; ++u) kv[u] = __builtin_bit_cast(VecE, *reinterpret_cast<const u32x4*>(kj + c + u * E));
 #pragma unroll
-        for (int e = 0; e < E; ++e) dot = fmaf(to_f32(qv[e]), to_f32(kv[e]), dot);
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) dot[r] = fmaf(to_f32(q[r][c + e]), to_f32(kv[e / E][e % E]), dot[r]);
+      }
+      for (; c < d; c += E) {
+        const VecE kv = __builtin_bit_cast(VecE, *reinterpret_cast<const u32x4*>(kj + c));
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int e = 0; e < E; ++e) dot[r] = fmaf(to_f32(q[r][c + e]), to_f32(kv[e]), dot[r]);
+      }
+    } else {
+      for (int c = 0; c < d; ++c) {
+        const float kv = to_f32(kj[c]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) dot[r] = fmaf(to_f32(q[r][c]), kv, dot[r]);
       }
     }
-  } else {
-    for (int c = 0; c < d; ++c) dot = fmaf(to_f32(qi[c]), to_f32(kj[c]), dot);
   }
-  srow[j] = scale * dot;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (i0 + r < N) S[(head + i0 + r) * N + j] = (causal && j > i0 + r) ? -INFINITY : scale * dot[r];
 }
 
 // Row r of S in place: max, sum of exp(s - max), then exp(s - max) / sum, each a strided pass
@@ -90,30 +108,48 @@ naive_softmax(float* __restrict__ S, int N, long long rows) {
   for (int j = lane; j < N; j += kWave) srow[j] = expf(srow[j] - mx) * rcp;
 }
 
-// O[h][i][c0 + lane] = sum over keys j of P[h][i][j] V[h][j][c0 + lane], for the wave's row i and
-// 64 head dims from c0. PIECES (N a multiple of 4, P 16-byte aligned): the wave reads its P row
-// four probabilities per load; the products are summed in the same order either way.
-template <typename T, bool PIECES>
+// O[h][i][c0 + lane] = sum over keys j of P[h][i][j] V[h][j][c0 + lane], for the wave's R rows i and
+// 64 head dims from c0, the keys in order. A V element serves the R rows, whose probabilities are the
+// same address in every lane (scalar loads; a row past N reads row N - 1 and is not stored). With
+// causal, the keys after the last of the rows, whose probabilities are zero, are left out.
+template <typename T, int R>
 __global__ void __launch_bounds__(256)
-naive_pv(const float* __restrict__ P, const T* __restrict__ V, T* __restrict__ O, int N, int d, int dim_blocks) {
-  const int unit = (int)blockIdx.x * 4 + (int)threadIdx.x / kWave;   // (query row, 64-dim block)
-  const int i = unit / dim_blocks;
+naive_pv(const float* __restrict__ P, const T* __restrict__ V, T* __restrict__ O, int N, int d, int causal,
+         int dim_blocks) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int unit = (int)blockIdx.x * 4 + wave;   // (R query rows, 64-dim block)
+  const int i0 = unit / dim_blocks * R;
   const int c = (unit % dim_blocks) * kWave + (int)threadIdx.x % kWave;
-  if (i >= N || c >= d) return;
+  if (i0 >= N || c >= d) return;
   const size_t head = (size_t)blockIdx.y * N;
-  const float* pi = P + (head + i) * N;
-  const T* vc = V + head * d + c;
-  float acc = 0.f;
-  if constexpr (PIECES) {
-    for (int j = 0; j < N; j += 4) {
-      const f32x4 p4 = *reinterpret_cast<const f32x4*>(pi + j);
+  const float* p[R];
+  float acc[R];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = fmaf(p4[e], to_f32(vc[(size_t)(j + e) * d]), acc);
-    }
-  } else {
-    for (int j = 0; j < N; ++j) acc = fmaf(pi[j], to_f32(vc[(size_t)j * d]), acc);
+  for (int r = 0; r < R; ++r) {
+    p[r] = P + (head + min(i0 + r, N - 1)) * N;
+    acc[r] = 0.f;
   }
-  O[(head + i) * d + c] = from_f32<T>(acc);
+  const T* vc = V + head * d + c;
+  const int n = causal ? min(N, i0 + R) : N;
+  constexpr int U = 16;   // keys per step: their loads are issued together
+  int j = 0;
+  for (; j + U <= n; j += U) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = to_f32(vc[(size_t)(j + u) * d]);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc[r] = fmaf(p[r][j + u], v[u], acc[r]);
+  }
+  for (; j < n; ++j) {
+    const float v = to_f32(vc[(size_t)j * d]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = fmaf(p[r][j], v, acc[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (i0 + r < N) O[(head + i0 + r) * d + c] = from_f32<T>(acc[r]);
 }
 
 // ------------------------------------------------------------------------------------ tiled

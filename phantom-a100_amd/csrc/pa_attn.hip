@@ -415,26 +415,36 @@ hipError_t launch_f16_terms(const void* q, const void* k, const void* v, void* o
 }
 
 // ------------------------------------------------------------------ unfused
+// Query rows a wave of a naive product takes: 8, which reuse each K / V element 8 times, where that
+// still leaves a wave for each of the chip's 1024 SIMDs, else 2 (a wave is then bound by its loads'
+// latency, and more of them run at once). Measured at 2 / 8 rows, us: fp32 8x16x1024 d = 128 5180 /
+// 2271, fp16 4x16x512 281 / 202, fp32 42x128 23.6 / 26.3, fp16 causal 2x600 d = 96 32 / 87; 4 rows lay
+// between the two, 16 were slower than 8.
+int naive_rows(long long n, long long col_blocks, long long bh) {
+  return (n + 7) / 8 * col_blocks * bh >= 4 * kCUs ? 8 : 2;
+}
 template <typename T>
 hipError_t launch_naive(const void* q, const void* k, const void* v, void* o, float* s, int bh, int n, int d,
                         int causal, hipStream_t stream) {
   const float scale = 1.f / sqrtf((float)d);
-  // Four waves per workgroup, one wave per (row, 64 columns); the heads in y.
+  // Four waves per workgroup, one wave per (rows, 64 columns); the heads in y.
   const long long key_blocks = (n + 63) / 64, dim_blocks = (d + 63) / 64;
-  const long long score_units = (long long)n * key_blocks, pv_units = (long long)n * dim_blocks;
+  const int score_rows = naive_rows(n, key_blocks, bh), pv_rows = naive_rows(n, dim_blocks, bh);
+  const long long score_units = ((long long)n + score_rows - 1) / score_rows * key_blocks;
+  const long long pv_units = ((long long)n + pv_rows - 1) / pv_rows * dim_blocks;
   const long long rows = (long long)n * bh;
   if (score_units > INT_MAX - 4 || pv_units > INT_MAX - 4 || (rows + 3) / 4 > INT_MAX)   // 32-bit unit indices
     return hipErrorInvalidConfiguration;
-  // Rows of whole 16-byte pieces, 16-byte aligned: the scores read them a piece per load.
-  const bool pieces = d * (int)sizeof(T) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(k) % 16 == 0;
-  auto scores = pieces ? pa::naive_scores<T, true> : pa::naive_scores<T, false>;
+  // Rows of whole 16-byte pieces, 16-byte aligned: the scores read K a piece per load.
+  const bool pieces = d * (int)sizeof(T) % 16 == 0 && reinterpret_cast<uintptr_t>(k) % 16 == 0;
+  auto scores = score_rows == 8 ? (pieces ? pa::naive_scores<T, true, 8> : pa::naive_scores<T, false, 8>)
+                                : (pieces ? pa::naive_scores<T, true, 2> : pa::naive_scores<T, false, 2>);
   hipLaunchKernelGGL(scores, dim3((unsigned)((score_units + 3) / 4), bh), dim3(256), 0, stream,
                      static_cast<const T*>(q), static_cast<const T*>(k), s, n, d, scale, causal, (int)key_blocks);
   hipLaunchKernelGGL(pa::naive_softmax, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, s, n, rows);
-  auto pv = n % 4 == 0 && reinterpret_cast<uintptr_t>(s) % 16 == 0 ? pa::naive_pv<T, true> : pa::naive_pv<T, false>;
+  auto pv = pv_rows == 8 ? pa::naive_pv<T, 8> : pa::naive_pv<T, 2>;
   hipLaunchKernelGGL(pv, dim3((unsigned)((pv_units + 3) / 4), bh), dim3(256), 0, stream, s,
-                     static_cast<const T*>(v), static_cast<T*>(o), n, d, (int)dim_blocks);
+                     static_cast<const T*>(v), static_cast<T*>(o), n, d, causal, (int)dim_blocks);
   return hipGetLastError();
 }
 

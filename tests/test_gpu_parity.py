@@ -432,6 +432,20 @@ def test_fused_tc_matches_rounded_p_model(path):
     assert err <= tol, f"vs the kernel model {err:.3e} > {tol:.1e} (reference algorithm vs float64: {e_ref:.2e})"
 
 
+# naive: 2 or 8 rows per wave (small and large grids), with whole and partial groups, 16-element steps
+# of dims and keys and their remainders.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("bh,n,d", [(1, 1, 1), (2, 9, 7), (1, 17, 20), (2, 65, 33), (600, 9, 16), (300, 33, 24),
+                                    (70, 127, 72), (260, 40, 65)])
+def test_naive_row_groups(bh, n, d, causal, dtype):
+    q, k, v = gpu_qkv(1, bh, n, d, dtype, seed=n + d)
+    ref = f64_reference_gpu(q, k, v, causal)
+    err = (cuda_attn.naive(q, k, v, causal).double() - ref).abs()
+    half_ulp = 0.0 if dtype == torch.float32 else 2.0 ** -11 * ref.abs()   # the output's rounding
+    assert (err <= F32_BAR + half_ulp).all()
+
+
 # fused with fp16 inputs: fp32 arithmetic on the fp16 matrix core (P in two fp16 terms).
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("bh,n", [(3, 1), (3, 31), (3, 64), (42, 65), (42, 128), (42, 129), (5, 191), (300, 192),
