@@ -48,7 +48,9 @@ enum pa_status {
 int pa_naive_fwd(const void* q, const void* k, const void* v, void* o, float* s,
                  int dtype, int64_t bh, int64_t n, int64_t d, int causal, void* stream);
 
-/* v2 tiled: LDS-tiled scores and P.V, one wave per softmax row; fp32 scores in workspace s.
+/* v2 tiled: two kernels (scores; softmax and P.V) with the fp32 scores in workspace s between them,
+ * or, for head dims that are not whole 16-byte rows up to 128, three. What s holds afterwards is not
+ * specified.
  * dtype: F32 or F16; any d >= 1.
  * Replaces attn::launch_tiled (csrc/kernels/tiled.cuh:108-117) and tiled_forward
  * (csrc/attn_tiled.cu:5-14). */

@@ -5,11 +5,11 @@
 //
 //   naive (/root/reference/csrc/kernels/naive.cuh:10-64): the same three passes (scores, softmax
 //         by row max / sum / normalise, P.V) as plain loops, a wave taking a few rows of each product.
-//   tiled (/root/reference/csrc/kernels/tiled.cuh:16-117): both products on the matrix core
-//         for fp16 inputs (scores at d a multiple of 16, P.V at d = 64 / 128) and for fp32 inputs
-//         at d = 64 / 128 (tiled_*_mfma, tiled_*_mfma_f32); otherwise 64x64 output tiles with 4x4
-//         register blocking per thread and LDS-staged operands. Softmax with one wave per row,
-//         the row held in registers up to 8192 keys (one read of S); longer rows take one
+//   tiled (/root/reference/csrc/kernels/tiled.cuh:16-117): rows of whole 16-byte pieces up to 128
+//         dims: the scores on the matrix core (tiled_scores_mfma), then softmax and P.V in one pass
+//         over them (tiled_softmax_pv). Other head dims and unaligned tensors: 64x64 output tiles
+//         with 4x4 register blocking per thread and LDS-staged operands. Softmax with one wave per
+//         row, the row held in registers up to 8192 keys (one read of S); longer rows take one
 //         workgroup per row, in register-held segments whose max the workgroup agrees on before
 //         their sums (one read of S up to 32768 keys, two beyond). Causal P.V skips key tiles
 //         right of the diagonal.
@@ -207,120 +207,352 @@ tiled_scores(const T* __restrict__ Q, const T* __restrict__ K, float* __restrict
   }
 }
 
-// S = scale * Q K^T on the matrix core, for fp16 storage and d = 16 * KSTEPS (the tiled_scores
-// result up to the order of the fp32 sums: products of fp16 values are exact in fp32). A 128 x 128
-// tile per workgroup, a 64 x 64 quarter per wave as 2 x 2 v_mfma_f32_32x32x16_f16 blocks, whose
-// operands are read straight from memory in the MFMA layout: lane l takes dims
-// 16 kk + 8 (l / 32) .. + 7 of row l % 32 of its 32-row block (16 bytes, rows 16-byte aligned);
-// rows past N read as zero through the buffer's range. Register r of a block holds row
-// 8 (r / 4) + 4 (l / 32) + r % 4 and column l % 32, so each store instruction writes 128
-// contiguous bytes of two rows. With causal, a quarter entirely right of the diagonal skips its
-// products and stores -inf.
-template <int KSTEPS>
-__global__ void __launch_bounds__(256)
-tiled_scores_mfma(const f16* __restrict__ Q, const f16* __restrict__ K, float* __restrict__ S, int N,
-                  float scale, int causal) {
-  constexpr int D = 16 * KSTEPS;
-  const int bh = blockIdx.z;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int r0 = blockIdx.y * 128 + (wave / 2) * 64;
-  const int c0 = blockIdx.x * 128 + (wave % 2) * 64;
-  const int lr = lane % 32, hk = lane / 32;
-  const uint32_t head_bytes = (uint32_t)((size_t)N * D * sizeof(f16));
-  const rsrc_t q_rs = make_rsrc(Q + (size_t)bh * N * D, head_bytes);
-  const rsrc_t k_rs = make_rsrc(K + (size_t)bh * N * D, head_bytes);
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = f32x16{};
-  if (!(causal && c0 > r0 + 63)) {
-    f16x8 a[KSTEPS][2], b[KSTEPS][2];
-#pragma unroll
-    for (int kk = 0; kk < KSTEPS; ++kk)
-#pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        a[kk][x] = __builtin_bit_cast(f16x8, load16(q_rs, (uint32_t)(((r0 + 32 * x + lr) * D + 16 * kk + 8 * hk) * 2)));
-        b[kk][x] = __builtin_bit_cast(f16x8, load16(k_rs, (uint32_t)(((c0 + 32 * x + lr) * D + 16 * kk + 8 * hk) * 2)));
-      }
-#pragma unroll
-    for (int kk = 0; kk < KSTEPS; ++kk)
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = mfma32x32x16(a[kk][rb], b[kk][cb], acc[rb][cb]);
-  }
-  float* Sb = S + (size_t)bh * N * N;
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = r0 + 32 * rb + 8 * (r / 4) + 4 * hk + r % 4;
-        const int j = c0 + 32 * cb + lr;
-        if (i < N && j < N) Sb[(size_t)i * N + j] = (causal && j > i) ? -INFINITY : acc[rb][cb][r] * scale;
-      }
-}
+// ---- Matrix-core form (head dims in whole 16-byte pieces up to 128, 16-byte aligned tensors): two
+// kernels, the scores and one pass over them for softmax and P.V together.
+//
+// What bounds it is the score workspace, 4 bytes per score and pass over it. Three kernels passed over
+// it four times (write, softmax read and write, P.V read); these two pass over it twice. The workspace
+// holds the raw dot products in the order in which the matrix core makes and takes them: each strip of
+// 32 query rows of a head (its last strip has the rb rows left) is a run of rb * N floats, the keys in
+// groups of 4 (the last group has the w keys left), so that the score of key k and the strip's row r is
+//     strip[rb * (k - k % 4) + w * r + k % 4],
+// and the strips fill a head's N * N floats exactly. A lane of a 32 x 32 S^T block (one query, groups
+// of 4 keys) then stores 16 contiguous bytes, a wave 1 KB per instruction, and the second kernel loads
+// its P^T operands the same way. (A strip starts 16-byte aligned only where N * N * head does: the
+// vectors are declared with an element's alignment.)
+//
+// Measured, three kernels -> two, us: fp16 4x16x2048 d = 64 980 -> 580 (scores 286, the rest 279: 3.8
+// TB/s each), causal 942 -> 394, 4x8x4096 1787 -> 945, 8x32x256 59 -> 39; fp32 4x16x2048 1350 -> 791
+// (both kernels also near the fp32 matrix core's rate). Rows and head dims that took the VALU kernels:
+// fp16 1x8x2000 d = 80 408 -> 63, 2x32x2047 d = 32 2022 -> 476, 1x1x4096 d = 96 641 -> 60; fp32
+// 1x16x333 d = 40 92 -> 20. Passes over a few heads at a time, whose scores stay in the memory-side
+// cache (192 MiB), gained 8 % at 4x16x2048 but lost up to 20 % on causal rows and smaller grids.
+// Against float64 the error is no larger (fp32 1x5x3392 d = 128 causal 5.2e-7 -> 3.8e-7; fp16 its
+// output's rounding).
+typedef float Score4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// S = scale * Q K^T on the fp32 matrix core (v_mfma_f32_32x32x2_f32) for fp32 storage and
-// D in {64, 128}; the tiled_scores result up to the order of its fp32 sums. 128 x 128 tile per
-// workgroup, 64 x 64 per wave as 2 x 2 blocks. The dot product's dims are walked in an order that
-// keeps every lane's reads contiguous: within each 64-dim chunk, k-step kk of lane l takes dim
-// 32 (l / 32) + kk of its row (l % 32 of the block), in Q and K alike, so a lane reads 32
-// consecutive floats (8 x 16 bytes) per row and chunk. Rows past N read as zero.
-template <int D>
+// Operands of an S^T = K Q^T block for the matrix core, read straight from memory in the MFMA layout;
+// rows past N and dims past d read as zero through the buffer's range.
+// fp16: one 32x32x16 step takes dims 16 kk + 8 (l / 32) .. + 7 of row l % 32.
+// fp32: 16 steps of 32x32x2 take dims 16 (l / 32) + 0 .. 15 of a 32-dim chunk, in Q and K alike.
+constexpr uint32_t kNoRow = 0x80000000u;   // an offset past every head (a head is below 2 GiB)
+
+// S^T blocks of 128 queries x 128 keys per workgroup, 64 x 64 per wave as 2 x 2 blocks of 32 x 32.
+// With causal, blocks whose keys all come after their queries are neither computed nor stored (the
+// second kernel does not read them).
+template <typename T>
 __global__ void __launch_bounds__(256)
-tiled_scores_mfma_f32(const float* __restrict__ Q, const float* __restrict__ K, float* __restrict__ S, int N,
-                      float scale, int causal) {
-  static_assert(D % 64 == 0, "64-dim chunks");
+tiled_scores_mfma(const T* __restrict__ Q, const T* __restrict__ K, float* __restrict__ S, int N, int d, int causal) {
   const int bh = blockIdx.z;
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int r0 = blockIdx.y * 128 + (wave / 2) * 64;
+  const int r0 = blockIdx.y * 128 + (wave / 2) * 64;   // first query, first key of the wave
   const int c0 = blockIdx.x * 128 + (wave % 2) * 64;
+  if (r0 >= N || c0 >= N || (causal && c0 > r0 + 63)) return;
   const int lr = lane % 32, hk = lane / 32;
-  const uint32_t head_bytes = (uint32_t)((size_t)N * D * sizeof(float));
-  const rsrc_t q_rs = make_rsrc(Q + (size_t)bh * N * D, head_bytes);
-  const rsrc_t k_rs = make_rsrc(K + (size_t)bh * N * D, head_bytes);
-  f32x16 acc[2][2];
+  const uint32_t head_bytes = (uint32_t)((size_t)N * d * sizeof(T));
+  const rsrc_t q_rs = make_rsrc(Q + (size_t)bh * N * d, head_bytes);
+  const rsrc_t k_rs = make_rsrc(K + (size_t)bh * N * d, head_bytes);
+  f32x16 acc[2][2];   // [key block][query block]
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+  for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = f32x16{};
-  if (!(causal && c0 > r0 + 63)) {
-#pragma unroll 1
-    for (int ch = 0; ch < D / 64; ++ch) {
-      f32x4 a[2][8], b[2][8];
+    for (int qb = 0; qb < 2; ++qb) acc[kb][qb] = f32x16{};
+  if constexpr (std::is_same<T, f16>::value) {
+    for (int c = 0; c < d; c += 32) {
+      f16x8 a[2][2], b[2][2];
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
+      for (int kk = 0; kk < 2; ++kk) {
+        const int col = c + 16 * kk + 8 * hk;
 #pragma unroll
-        for (int v = 0; v < 8; ++v) {
-          const uint32_t col = (uint32_t)(64 * ch + 32 * hk + 4 * v);
-          a[x][v] = __builtin_bit_cast(f32x4, load16(q_rs, (uint32_t)((r0 + 32 * x + lr) * D + col) * 4));
-          b[x][v] = __builtin_bit_cast(f32x4, load16(k_rs, (uint32_t)((c0 + 32 * x + lr) * D + col) * 4));
+        for (int x = 0; x < 2; ++x) {
+          a[kk][x] = __builtin_bit_cast(f16x8, load16(k_rs, col < d ? (uint32_t)((c0 + 32 * x + lr) * d + col) * 2 : kNoRow));
+          b[kk][x] = __builtin_bit_cast(f16x8, load16(q_rs, col < d ? (uint32_t)((r0 + 32 * x + lr) * d + col) * 2 : kNoRow));
         }
+      }
 #pragma unroll
-      for (int kk = 0; kk < 32; ++kk)
+      for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
+        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int cb = 0; cb < 2; ++cb)
-            acc[rb][cb] = mfma32x32x2(a[rb][kk / 4][kk % 4], b[cb][kk / 4][kk % 4], acc[rb][cb]);
+          for (int qb = 0; qb < 2; ++qb) acc[kb][qb] = mfma32x32x16(a[kk][kb], b[kk][qb], acc[kb][qb]);
+    }
+  } else {
+    for (int c = 0; c < d; c += 32) {
+      f32x4 a[2][4], b[2][4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int col = c + 16 * hk + 4 * v;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          a[x][v] = __builtin_bit_cast(f32x4, load16(k_rs, col < d ? (uint32_t)((c0 + 32 * x + lr) * d + col) * 4 : kNoRow));
+          b[x][v] = __builtin_bit_cast(f32x4, load16(q_rs, col < d ? (uint32_t)((r0 + 32 * x + lr) * d + col) * 4 : kNoRow));
+        }
+      }
+#pragma unroll
+      for (int kk = 0; kk < 16; ++kk)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int qb = 0; qb < 2; ++qb)
+            acc[kb][qb] = mfma32x32x2(a[kb][kk / 4][kk % 4], b[qb][kk / 4][kk % 4], acc[kb][qb]);
     }
   }
-  float* Sb = S + (size_t)bh * N * N;
+  // Register r of a block holds key 8 (r / 4) + 4 hk + r % 4 and query lr.
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+  for (int qb = 0; qb < 2; ++qb) {
+    const int i0 = r0 + 32 * qb;
+    const int rb = min(32, N - i0);
+    if (lr >= rb) continue;
+    float* strip = S + (size_t)bh * N * N + (size_t)i0 * N;
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = r0 + 32 * rb + 8 * (r / 4) + 4 * hk + r % 4;
-        const int j = c0 + 32 * cb + lr;
-        if (i < N && j < N) Sb[(size_t)i * N + j] = (causal && j > i) ? -INFINITY : acc[rb][cb][r] * scale;
+      for (int g = 0; g < 4; ++g) {
+        const int key = c0 + 32 * kb + 8 * g + 4 * hk, w = N - key;
+        if (w >= 4) {
+          Score4 x;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = acc[kb][qb][4 * g + e];
+          *reinterpret_cast<Score4*>(strip + rb * key + 4 * lr) = x;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 3; ++e)
+            if (e < w) strip[rb * key + w * lr + e] = acc[kb][qb][4 * g + e];
+        }
       }
+  }
 }
 
+// O = softmax(scale S) V in one pass over the strips: the fused kernels' online softmax (fa_mfma.hpp)
+// with the S^T blocks loaded instead of computed. A wave owns a strip of 32 query rows; per tile of BN
+// keys, the row max (m raised, and l and O rescaled, only when a row's max has outgrown it by 2^8),
+// P = 2^(S c - m), and O^T += V^T P^T on the matrix core from a V tile in LDS.
+// fp16 V: P (taken 2^7 larger, at most 2^15) as two fp16 terms, 22 bits, on the fp16 matrix core; V^T
+// read with ds_read_b64_tr_b16. fp32 V: P and V as they are on the fp32 matrix core, whose two k-slots
+// take the keys that the two lane halves hold.
+// V goes to LDS with direct loads (two stages), the next tile's scores to registers, during the current
+// tile; several workgroups per CU keep enough of both in flight. KS > 1: the keys are dealt tile by
+// tile to KS waves of one strip, each with its own V stages, (m, l, O) merged at the end, for grids
+// that would leave CUs without a workgroup.
+template <typename T, int NDB, int KS>
+__global__ void __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(KS == 1 && NDB <= 2 ? 4 : 3)))
+tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __restrict__ O, int N, int d, float scale_log2,
+                 int causal) {
+  constexpr bool HALF = std::is_same<T, f16>::value;
+  constexpr int NQ = 4 / KS, BN = KS == 1 ? 64 : 32;
+  constexpr int DP = NDB <= 2 ? 64 : 128;           // dims of a V row in LDS
+  constexpr int RB = DP * (int)sizeof(T), CR = RB / 16, EPC = 16 / (int)sizeof(T);
+  constexpr int TILE_BYTES = BN * RB, THREADS = NQ * kWave;
+  constexpr int CPT = BN * CR / THREADS;            // 16-byte V chunks per thread per tile
+  constexpr int NG = BN / 8;                        // groups of 4 keys per lane and tile
+  constexpr float kLazyLog2 = 8.f, kTermShift = HALF ? 7.f : 0.f;
+  __shared__ __attribute__((aligned(1024))) unsigned char v_lds[KS * 2 * TILE_BYTES];
+  __shared__ float red_ml[KS > 1 ? (KS - 1) * 2 * kWave : 1];
+  const int bh = blockIdx.y;
+  const int g = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / THREADS);   // key group
+  const int tid = (int)threadIdx.x % THREADS, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lq = lane % 32, hi = lane / 32;
+  const int qblk = causal ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x;   // longest causal rows first
+  const int q0 = qblk * 32 * NQ, i0 = q0 + 32 * wave, qrow = i0 + lq;
+  const int rb = min(32, N - i0);                   // rows of the wave's strip (none: rb <= 0)
+  const float* strip = S + (size_t)bh * N * N + (size_t)min(i0, N - 1) * N;
+  const rsrc_t v_rs = make_rsrc(V + (size_t)bh * N * d, (uint32_t)((size_t)N * d * sizeof(T)));
+  unsigned char* lds = v_lds + g * 2 * TILE_BYTES;
+
+  // V tile: chunk swizzle by row. fp16: the fused kernels'. fp32: rows 4 apart, read by the two lane
+  // halves at the same dim, differ by half the banks.
+  auto swz = [](int row) { return HALF ? v_swz<CR>(row) : 8 * ((row >> 2) & 1); };
+  uint32_t v_src[CPT];
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int slot = i * THREADS + tid, row = slot / CR, c = (slot % CR) ^ swz(row);
+    v_src[i] = c * EPC < d ? (uint32_t)(row * d + c * EPC) * (uint32_t)sizeof(T) : kNoRow;
+  }
+  auto load_v = [&](int stage, int k0) {
+#pragma unroll
+    for (int i = 0; i < CPT; ++i)
+      load16_to_lds(v_rs, lds + stage * TILE_BYTES + (i * THREADS + wave * kWave) * 16, v_src[i],
+                    (uint32_t)k0 * (uint32_t)(d * sizeof(T)));
+  };
+  int v_addr[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) {
+    if constexpr (HALF) {   // the transposed reads of fa_mfma.hpp
+      const int g16 = lane / 16, i16 = lane % 16, v_row = hi * 4 + i16 / 4, v_cl = 2 * (g16 % 2) + (i16 % 4) / 2;
+      v_addr[db] = v_row * RB + (((4 * db + v_cl) ^ swz(v_row)) * 16) + 8 * (i16 % 2);
+    } else {                // V[4 hi][32 db + lq]; rows 8 further on have the same swizzle
+      v_addr[db] = 4 * hi * RB + (((8 * db + lq / 4) ^ swz(4 * hi)) * 16) + 4 * (lq % 4);
+    }
+  }
+  // Scores of a tile: group i of the lane is keys k0 + 8 i + 4 hi .. + 3 of its row. Rows past the
+  // strip read its last row (not stored); keys past N are not read.
+  const int pitch = max(rb, 1), lrow = min(lq, pitch - 1);
+  const uint32_t s_off = (uint32_t)(pitch * 4 * hi + 4 * lrow);   // this lane's offset from key group 8 i
+  auto load_s = [&](f32x4 (&x)[NG], int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NG; ++i) x[i] = *reinterpret_cast<const Score4*>(strip + pitch * (k0 + 8 * i) + s_off);
+  };
+  // The tile that N ends in, an element per load (keys past N read the strip's first score; masked).
+  auto load_last = [&](f32x4 (&x)[NG], int k0) __attribute__((always_inline)) {
+    int w0 = N - k0 - 4 * hi;   // keys left from the lane's first one
+    asm volatile("" : "+v"(w0));
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      const int w = w0 - 8 * i;
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = strip[e < w ? pitch * (N - w) + min(w, 4) * lrow + e : 0];
+      x[i] = f32x4{y[0], y[1], y[2], y[3]};
+    }
+  };
+
+  float m_run = -INFINITY, l_run = 0.f;
+  f32x16 o[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) o[db] = f32x16{};
+  const int kv_end = causal ? min(N, q0 + 32 * NQ) : N;
+  const int ntiles = (kv_end + BN - 1) / BN, nit = (ntiles + KS - 1) / KS;
+  const int wave_end = rb <= 0 ? 0 : causal ? min(N, i0 + 32) : N;   // keys that the wave's rows see
+  const int wave_tiles = (wave_end + BN - 1) / BN;
+  const int clean_tiles = causal ? min(N, i0 + 1) / BN : N / BN;       // of these, without a mask
+
+  auto compute = [&](f32x4 (&x)[NG], const unsigned char* vs, int t) __attribute__((always_inline)) {
+    if (t >= clean_tiles) {
+      // Key t BN + 8 i + 4 hi + e is visible iff 8 i + e <= lim (hidden from the compiler, which would
+      // keep the limit of every element in registers).
+      int lim = (causal ? min(N - 1, qrow) : N - 1) - t * BN - 4 * hi;
+      asm volatile("" : "+v"(lim));
+#pragma unroll
+      for (int i = 0; i < NG; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (8 * i + e > lim) x[i][e] = -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NG; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mx = fmaxf(mx, x[i][e]);
+    const float m_new = fmaxf(m_run, half_max(mx) * scale_log2);
+    if (__builtin_amdgcn_ballot_w64(m_new > m_run + kLazyLog2) != 0) {
+      const float alpha = m_new > m_run ? exp2_fast(m_run - m_new) : 1.f;   // m_run = -inf -> 0
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) o[db] *= alpha;
+    }
+    const float nm = m_run == -INFINITY ? 0.f : kTermShift - m_run;   // no visible key so far: P = 0
+    float sum = 0.f;                                                  // the tile's sum, then one add to l
+#pragma unroll
+    for (int i = 0; i < NG; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[i][e] = exp2_fast(fmaf(x[i][e], scale_log2, nm));
+        sum += x[i][e];
+      }
+    l_run += sum;
+#pragma unroll
+    for (int ks = 0; ks < BN / 16; ++ks) {
+      if constexpr (HALF) {
+        f16x8 ph, pl;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float p = x[2 * ks + j / 4][j % 4];
+          ph[j] = (f16)p;
+          pl[j] = (f16)(p - (float)ph[j]);
+        }
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+          const unsigned char* p0 = vs + ks * 16 * RB + v_addr[db];
+          const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0));
+          const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0 + 8 * RB));
+          const f16x8 a = __builtin_bit_cast(f16x8, i16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]});
+          o[db] = mfma32x32x16(a, pl, o[db]);
+          o[db] = mfma32x32x16(a, ph, o[db]);
+        }
+      } else {
+#pragma unroll
+        for (int i = 2 * ks; i < 2 * ks + 2; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+              o[db] = mfma32x32x2(*reinterpret_cast<const float*>(vs + (8 * i + e) * RB + v_addr[db]), x[i][e], o[db]);
+      }
+    }
+  };
+
+  // Key group g's iteration j is tile j KS + g. At the top of an iteration its tile has landed and
+  // every wave is done with the stage that the next tile goes to.
+  const int full_tiles = min(wave_tiles, N / BN);
+  f32x4 x[NG], xn[NG];
+  if (g < ntiles) load_v(0, g * BN);
+  if (g < full_tiles) load_s(x, g * BN);
+#pragma unroll 1
+  for (int j = 0; j < nit; ++j) {
+    const int t = j * KS + g;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (t + KS < ntiles) load_v((j + 1) & 1, (t + KS) * BN);
+    if (t + KS < full_tiles) load_s(xn, (t + KS) * BN);
+    if (t < wave_tiles) {
+      if (t >= full_tiles) load_last(x, t * BN);
+      compute(x, lds + (j & 1) * TILE_BYTES, t);
+    }
+#pragma unroll
+    for (int i = 0; i < NG; ++i) x[i] = xn[i];
+  }
+  float l = half_sum(l_run);
+  if constexpr (KS > 1) {
+    static_assert((KS - 1) * NDB * 16 * kWave * 4 <= KS * 2 * TILE_BYTES, "merge through the stages");
+    __syncthreads();
+    if (g > 0) {
+      float* red_o = reinterpret_cast<float*>(v_lds) + (g - 1) * NDB * 16 * kWave;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red_o[(db * 16 + r) * kWave + lane] = o[db][r];
+      red_ml[(g - 1) * 2 * kWave + lane] = m_run;
+      red_ml[(g - 1) * 2 * kWave + kWave + lane] = l;
+    }
+    __syncthreads();
+    if (g > 0) return;
+#pragma unroll 1
+    for (int x = 0; x < KS - 1; ++x) {
+      const float* red_o = reinterpret_cast<const float*>(v_lds) + x * NDB * 16 * kWave;
+      const float m1 = red_ml[x * 2 * kWave + lane], l1 = red_ml[x * 2 * kWave + kWave + lane];
+      const float m = fmaxf(m_run, m1);
+      const float sc0 = m_run == -INFINITY ? 0.f : exp2_fast(m_run - m);
+      const float sc1 = m1 == -INFINITY ? 0.f : exp2_fast(m1 - m);   // a group without visible keys adds nothing
+      m_run = m;
+      l = sc0 * l + sc1 * l1;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] = sc0 * o[db][r] + sc1 * red_o[(db * 16 + r) * kWave + lane];
+    }
+  }
+  // Register r of block db holds dim 32 db + 8 (r / 4) + 4 hi + r % 4 of query qrow.
+  if (qrow < N) {
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const float inv = 1.f / l;
+    T* orow = O + ((size_t)bh * N + qrow) * d;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        const int c = 32 * db + 8 * g4 + 4 * hi;
+        T4 w;
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) w[rr] = from_f32<T>(o[db][g4 * 4 + rr] * inv);
+        if (c < d) *reinterpret_cast<T4*>(orow + c) = w;
+      }
+  }
+}
+
+// ---- General form (any head dim): the scores row by row in the workspace, softmax in place, P.V.
 // One wave per row, the whole row held in registers (rows of at most 64 * VPL keys): S is read
 // once and P written once, 8 bytes per score (the naive softmax reads S three times). The max
 // first, then the sum of exp(x - max) kept in place, then P = e / sum; element j of the row sits in
@@ -419,203 +651,6 @@ tiled_softmax_segments(float* __restrict__ S, int N) {
   } else {
     for (int j = t; j < N; j += 256) row[j] = expf(row[j] - m) * inv;
   }
-}
-
-// O = P V on the matrix core for fp16 V with D in {64, 128} (the fused kernel's V operand path),
-// computed transposed as O^T += V^T P^T per 16-key step with v_mfma_f32_32x32x16_f16: A = V^T,
-// read from a swizzled LDS tile of 64 keys with ds_read_b64_tr_b16; B = P^T, lane l taking the 8
-// probabilities of its query row l % 32 at the keys the V reads pair with them (two runs of 4
-// consecutive keys) straight from the fp32 workspace. P is fed as two fp16 terms of 1024 P
-// (hi = round(1024 P), lo = round(1024 P - hi)): ~22 significant bits while lo is a normal fp16
-// (|lo| ~ 2^-11 |hi| >= 2^-14, i.e. P >= ~2^-13); below that lo lands on fp16's subnormal spacing
-// 2^-24, so the pair is off by at most 2^-25 in 1024 P, 2^-35 in P. Both products are exact in
-// fp32 and summed in fp32; O is scaled back by 2^-10. 128 queries per workgroup (32 per wave),
-// two V stages; the next tile's V (to LDS) and P (to registers) load during the current one.
-// Reads past the head (query or key rows past N) return zero through the buffers' ranges, and
-// keys past N meet zero V rows. With causal, keys after the block's last query are skipped (their
-// P is zero).
-template <int D>
-__global__ void __launch_bounds__(256)
-tiled_pv_mfma(const float* __restrict__ P, const f16* __restrict__ V, f16* __restrict__ O, int N, int causal) {
-  constexpr int BN = 64, THREADS = 256, NDB = D / 32, CR = D / 8, RB = D * 2;
-  constexpr int TILE_BYTES = BN * RB;
-  constexpr int CPT = BN * CR / THREADS;   // 16-byte V chunks per thread per tile
-  static_assert(D == 64 || D == 128, "V layout of the fused kernel");
-  __shared__ __attribute__((aligned(1024))) unsigned char v_lds[2 * TILE_BYTES];
-  const int bh = blockIdx.y;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  const int lq = lane % 32, hi = lane / 32;
-  const int q0 = blockIdx.x * 128;
-  const int qrow = q0 + wave * 32 + lq;
-  const rsrc_t v_rs = make_rsrc(V + (size_t)bh * N * D, (uint32_t)((size_t)N * D * sizeof(f16)));
-  const rsrc_t p_rs = make_rsrc(P + (size_t)bh * N * N, (uint32_t)((size_t)N * N * sizeof(float)));
-  uint32_t v_src[CPT];
-#pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    const int slot = i * THREADS + tid;
-    const int row = slot / CR, pc = slot % CR;
-    v_src[i] = (uint32_t)(row * RB + ((pc ^ v_swz<CR>(row)) * 16));
-  }
-  auto load_v = [&](int stage, int k0) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i)
-      load16_to_lds(v_rs, v_lds + stage * TILE_BYTES + (i * THREADS + wave * kWave) * 16, v_src[i], (uint32_t)(k0 * RB));
-  };
-  const int g16 = lane / 16, i16 = lane % 16;
-  const int v_row = hi * 4 + i16 / 4;
-  const int v_cl = 2 * (g16 % 2) + (i16 % 4) / 2;
-  int v_addr[NDB];
-#pragma unroll
-  for (int db = 0; db < NDB; ++db)
-    v_addr[db] = v_row * RB + (((4 * db + v_cl) ^ v_swz<CR>(v_row)) * 16) + 8 * (i16 % 2);
-  // P^T operands of one 64-key tile: for 16-key step ks, k-slot j of this lane holds key
-  // 16 ks + 8 (j / 4) + 4 hi + j % 4 of its query row, the key order in which the transposed
-  // V reads hand out the A operand (rows 4 hi .. 4 hi + 3, then 8 + 4 hi .. 8 + 4 hi + 3).
-  auto load_p = [&](u32x4 (&pr)[8], int k0) {
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        pr[2 * ks + h] = load16(p_rs, (uint32_t)(((size_t)qrow * N + k0 + 16 * ks + 8 * h + 4 * hi) * sizeof(float)));
-  };
-  f32x16 acc[NDB];
-#pragma unroll
-  for (int db = 0; db < NDB; ++db) acc[db] = f32x16{};
-  const int k_end = causal ? min(N, q0 + 128) : N;
-  const int ntiles = (k_end + BN - 1) / BN;
-  u32x4 pc[8], pn[8];
-  load_v(0, 0);
-  load_p(pc, 0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    if (t + 1 < ntiles) {
-      load_v((t + 1) & 1, (t + 1) * BN);
-      load_p(pn, (t + 1) * BN);
-    }
-    const unsigned char* vs = v_lds + (t & 1) * TILE_BYTES;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      f16x8 ph, pl;
-      // (the whole u32x4 is bit-cast to f32x4: casting one element of a loaded u32x4 to float
-      // miscompiles with this hipcc, every element then reading element 0)
-      const f32x4 p4[2] = {__builtin_bit_cast(f32x4, pc[2 * ks]), __builtin_bit_cast(f32x4, pc[2 * ks + 1])};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float x = 1024.f * p4[j / 4][j % 4];
-        const f16 h = (f16)x;
-        ph[j] = h;
-        pl[j] = (f16)(x - (float)h);
-      }
-#pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        const unsigned char* p0 = vs + ks * 16 * RB + v_addr[db];
-        const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0));
-        const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0 + 8 * RB));
-        const f16x8 a = __builtin_bit_cast(f16x8, i16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]});
-        acc[db] = mfma32x32x16(a, ph, acc[db]);
-        acc[db] = mfma32x32x16(a, pl, acc[db]);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) pc[i] = pn[i];
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  }
-  // Register r of block db holds dim 32 db + 8 (r / 4) + 4 hi + r % 4 of query qrow.
-  if (qrow < N) {
-    f16* orow = O + ((size_t)bh * N + qrow) * D;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        typedef f16 F16x4 __attribute__((ext_vector_type(4)));
-        F16x4 w;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) w[rr] = (f16)(acc[db][g4 * 4 + rr] * (1.f / 1024.f));
-        *reinterpret_cast<F16x4*>(orow + db * 32 + g4 * 8 + hi * 4) = w;
-      }
-  }
-}
-
-// O = P V on the fp32 matrix core for fp32 V and D in {64, 128}: A = P (lane l: 32 consecutive
-// probabilities of its query row l % 32 per 64-key tile, the keys of k-step kk being
-// 32 (l / 32) + kk, read straight from the workspace), B = V from a 64-key LDS tile (lane l reads
-// key 32 (l / 32) + kk, dim l % 32 of its 32-dim block). 128 queries per workgroup, 32 per wave;
-// the next tile's V (to LDS) and P (to registers) load during the current one. Reads past the
-// head return zero; keys past N meet zero V rows. With causal, keys after the block's last query
-// are skipped.
-template <int D>
-__global__ void __launch_bounds__(256)
-tiled_pv_mfma_f32(const float* __restrict__ P, const float* __restrict__ V, float* __restrict__ O, int N, int causal) {
-  constexpr int BN = 64, THREADS = 256, NDB = D / 32;
-  constexpr int ROW = D + 4;                       // LDS row pitch in floats (padding spreads banks)
-  static_assert(D == 64 || D == 128, "head dim");
-  __shared__ __attribute__((aligned(16))) float v_lds[2][BN * ROW];
-  const int bh = blockIdx.y;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  const int lq = lane % 32, hi = lane / 32;
-  const int q0 = blockIdx.x * 128;
-  const int qrow = q0 + wave * 32 + lq;
-  const rsrc_t v_rs = make_rsrc(V + (size_t)bh * N * D, (uint32_t)((size_t)N * D * sizeof(float)));
-  const rsrc_t p_rs = make_rsrc(P + (size_t)bh * N * N, (uint32_t)((size_t)N * N * sizeof(float)));
-  // V tile: 64 keys x D floats, 16 bytes per thread per load, rows of D / 4 chunks.
-  constexpr int CH = BN * D / 4 / THREADS;
-  auto load_v = [&](u32x4 (&vr)[CH], int k0) {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int slot = i * THREADS + tid, row = slot / (D / 4), c4 = slot % (D / 4);
-      vr[i] = load16(v_rs, (uint32_t)(((k0 + row) * D + 4 * c4) * 4));
-    }
-  };
-  auto store_v = [&](const u32x4 (&vr)[CH], int stage) {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int slot = i * THREADS + tid, row = slot / (D / 4), c4 = slot % (D / 4);
-      *reinterpret_cast<f32x4*>(&v_lds[stage][row * ROW + 4 * c4]) = __builtin_bit_cast(f32x4, vr[i]);
-    }
-  };
-  auto load_p = [&](u32x4 (&pr)[8], int k0) {
-#pragma unroll
-    for (int v = 0; v < 8; ++v)
-      pr[v] = load16(p_rs, (uint32_t)(((size_t)qrow * N + k0 + 32 * hi + 4 * v) * sizeof(float)));
-  };
-  f32x16 acc[NDB];
-#pragma unroll
-  for (int db = 0; db < NDB; ++db) acc[db] = f32x16{};
-  const int k_end = causal ? min(N, q0 + 128) : N;
-  const int ntiles = (k_end + BN - 1) / BN;
-  u32x4 vr[CH], pc[8], pn[8];
-  load_v(vr, 0);
-  load_p(pc, 0);
-  store_v(vr, 0);
-  __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const bool more = t + 1 < ntiles;
-    if (more) {
-      load_v(vr, (t + 1) * BN);
-      load_p(pn, (t + 1) * BN);
-    }
-    const float* vs = v_lds[t & 1];
-#pragma unroll
-    for (int kk = 0; kk < 32; ++kk) {
-      const float a = __builtin_bit_cast(f32x4, pc[kk / 4])[kk % 4];
-#pragma unroll
-      for (int db = 0; db < NDB; ++db) acc[db] = mfma32x32x2(a, vs[(32 * hi + kk) * ROW + 32 * db + lq], acc[db]);
-    }
-    if (more) store_v(vr, (t + 1) & 1);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) pc[i] = pn[i];
-    __syncthreads();
-  }
-  // Register r of block db holds query 8 (r / 4) + 4 hi + r % 4 of the wave and dim 32 db + l % 32.
-#pragma unroll
-  for (int db = 0; db < NDB; ++db)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int q = q0 + wave * 32 + 8 * (r / 4) + 4 * hi + r % 4;
-      if (q < N) O[((size_t)bh * N + q) * D + 32 * db + lq] = acc[db][r];
-    }
 }
 
 // O[i0:i0+64, c0:c0+64] = P_rows . V_cols; with causal, P is zero right of the diagonal so

@@ -9,7 +9,7 @@ messages. Underneath, every entry point calls hand-written HIP kernels in libpha
 through its C ABI (include/phantom_attn.h); there is no CPU or PyTorch fallback.
 
     naive        3 kernels, fp32 N x N scores in a workspace        any d, fp32/fp16
-    tiled        LDS-tiled scores / P.V, one wave per softmax row     any d, fp32/fp16
+    tiled        matrix-core scores, then softmax and P.V over them   any d, fp32/fp16
     fused        fused online softmax, fp32 arithmetic on MFMA        d=64, fp32/fp16
     fused_tuned  fp16 MFMA fused kernel at a chosen (br, bc) tile and 1 or 2 LDS stages
     fused_tc     fp16/bf16 MFMA fused kernel                          d=64 or 128
@@ -100,7 +100,7 @@ def naive(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fals
 
 
 def tiled(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = False) -> torch.Tensor:
-    """v2: LDS-tiled matmuls and a wave-per-row softmax, N x N scores still in HBM."""
+    """v2: matrix-core products with the N x N scores still in HBM between them."""
     return _unfused("pa_tiled_fwd", "tiled_forward", q, k, v, causal)
 
 

@@ -280,6 +280,27 @@ def test_tiled_fp16_head_dims(d, n, causal):
     assert max_err(out, f64_reference_gpu(q, k, v, causal)) <= 2e-3
 
 
+@pytest.mark.parametrize("shape", [
+    (1, 1, 1, 8), (1, 3, 31, 32), (2, 2, 33, 40), (1, 2, 66, 64), (1, 2, 131, 96), (1, 1, 383, 128),   # split keys
+    (1, 260, 99, 40), (1, 130, 130, 104), (1, 64, 515, 64)])                                            # 128-row blocks
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("causal", [False, True])
+def test_tiled_strips(shape, dtype, causal):
+    """The matrix-core form of tiled against float64: every N % 4, partial strips and key tiles, odd
+    heads (whose strips are not 16-byte aligned), head dims that are not whole 32-dim blocks, split and
+    unsplit keys; the workspace holds exactly B*H*N*N scores, and what follows it stays."""
+    b, h, n, d = shape
+    code = {torch.float32: _native.DTYPE_F32, torch.float16: _native.DTYPE_F16}[dtype]
+    q, k, v = gpu_qkv(b, h, n, d, dtype, seed=21)
+    s = torch.full((b * h * n * n + 64,), 7.0, dtype=torch.float32, device="cuda")
+    o = torch.empty_like(q)
+    rc = _native.lib().pa_tiled_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), s.data_ptr(), code, b * h, n,
+                                    d, int(causal), torch.cuda.current_stream().cuda_stream)
+    _native.check(rc, "tiled_forward")
+    assert max_err(o.double(), f64_reference_gpu(q, k, v, causal)) <= (F32_BAR if dtype == torch.float32 else 2e-3)
+    assert torch.all(s[b * h * n * n:] == 7.0)
+
+
 @pytest.mark.parametrize("name", ["fused", "fused_vec"])
 def test_fused_rejects_unsupported_head_dim(name):
     q, k, v = gpu_qkv(1, 1, 64, 128, torch.float16)
