@@ -70,7 +70,8 @@ int pa_tiled_fwd_noalloc(const void* q, const void* k, const void* v, void* o,
                          int dtype, int64_t bh, int64_t n, int64_t d, int causal, void* stream);
 
 /* v3 fused: online softmax with fp32 arithmetic throughout: fp32 inputs on the fp32 matrix core, P
- * kept in fp32, or on larger grids on the bf16 one with every operand in three bf16 terms; fp16 inputs on the fp16 matrix core, whose products are exact, with P in two fp16
+ * kept in fp32, or on larger grids on the 16-bit one with every operand in two fp16 or three bf16
+ * terms (24 significant bits); fp16 inputs on the fp16 matrix core, whose products are exact, with P in two fp16
  * terms of 22 significant bits (both with errors against float64
  * below the fp32 matrix core's). fp16 calls
  * take fused_tc's launch forms, and pa_set_persistent() applies to them.
