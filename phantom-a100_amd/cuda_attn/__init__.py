@@ -36,11 +36,11 @@ _LDS_NEED: dict = {}
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _stream_ptr(t: torch.Tensor) -> int:
+def _stream_ptr(device: torch.device) -> int:
     if _raw_stream is not None:
-        idx = t.device.index
+        idx = device.index
         return _raw_stream(torch.cuda.current_device() if idx is None else idx)
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def _lds_need(key, fn, *args) -> int:
@@ -75,12 +75,14 @@ def _call(fn_name: str, err_name: str, device: torch.device, *args) -> None:
     fn = _FNS.get(fn_name)
     if fn is None:
         fn = _FNS[fn_name] = getattr(_native.lib(), fn_name)
-    if device.index is None or device.index == _get_device():
+    index = device.index
+    if index is None or index == _get_device():
         rc = fn(*args)
     else:
         with torch.cuda.device(device):
             rc = fn(*args)
-    _native.check(rc, err_name)
+    if rc:
+        _native.check(rc, err_name)
 
 
 def _unfused(fn_name: str, err_name: str, q, k, v, causal: bool) -> torch.Tensor:
@@ -90,7 +92,7 @@ def _unfused(fn_name: str, err_name: str, q, k, v, causal: bool) -> torch.Tensor
     s = torch.empty((q.shape[0], q.shape[1], n, n), dtype=torch.float32, device=q.device)
     o = torch.empty_like(q)
     _call(fn_name, err_name, q.device, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), s.data_ptr(),
-          _DTYPE_CODE[q.dtype], bh, n, d, int(bool(causal)), _stream_ptr(q))
+          _DTYPE_CODE[q.dtype], bh, n, d, int(bool(causal)), _stream_ptr(q.device))
     return o
 
 
@@ -108,13 +110,15 @@ def fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fals
           out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """v3: one fused kernel with online softmax in fp32 arithmetic. Requires d == 64."""
     _checks.check_inputs(q, k, v)
-    _checks.check_head_dim("fused_forward", q, (64,))
+    b, h, n, d = q.shape
+    dtype, device = q.dtype, q.device
+    if d != 64:
+        _checks.check_head_dim("fused_forward", q, (64,))
     _checks.check_float_half("fused_forward", q)
-    od = _checks.resolve_out_dtype("fused_forward", q, out_dtype)
-    bh, n, d = _bhnd(q)
-    o = (torch.empty_like(q) if od == q.dtype else torch.empty_like(q, dtype=od))
-    _call("pa_fused_fwd", "fused_forward", q.device, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-          _DTYPE_CODE[q.dtype], _DTYPE_CODE[od], bh, n, d, int(bool(causal)), _stream_ptr(q))
+    od = dtype if out_dtype is None else _checks.resolve_out_dtype("fused_forward", q, out_dtype)
+    o = torch.empty_like(q) if od is dtype else torch.empty_like(q, dtype=od)
+    _call("pa_fused_fwd", "fused_forward", device, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+          _DTYPE_CODE[dtype], _DTYPE_CODE[od], b * h, n, d, 1 if causal else 0, _stream_ptr(device))
     return o
 
 
@@ -137,7 +141,7 @@ def fused_tuned(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool 
     o = (torch.empty_like(q) if od == q.dtype else torch.empty_like(q, dtype=od))
     _call("pa_fused_tuned_fwd", "fused_tuned", q.device, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
           _native.DTYPE_F16, _DTYPE_CODE[od], bh, n, d, int(bool(causal)), int(bool(double_buffer)), int(br), int(bc),
-          _stream_ptr(q))
+          _stream_ptr(q.device))
     return o
 
 
@@ -168,15 +172,22 @@ def fused_tc(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = F
     on non-causal rows: the persistent kernel starts a rescale on the packed maximum of the rounded
     probabilities, the per-block one on the row maximum; both within the fp16 bar)."""
     _checks.check_inputs(q, k, v)
-    _checks.check_tc(q, k, v)
-    od = _checks.resolve_out_dtype("fused_tc", q, out_dtype)
-    d, code = q.shape[3], _DTYPE_CODE[q.dtype]
-    need = _lds_need(("tc", d, code), _native.lib().pa_fused_tc_lds_bytes, d, code)
-    _checks.check_lds("fused_tc", need, _lds_limit(q))
-    bh, n, d = _bhnd(q)
-    o = (torch.empty_like(q) if od == q.dtype else torch.empty_like(q, dtype=od))
-    _call("pa_fused_tc_fwd", "fused_tc", q.device, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-          _DTYPE_CODE[q.dtype], _DTYPE_CODE[od], bh, n, d, int(bool(causal)), _stream_ptr(q))
+    b, h, n, d = q.shape
+    dtype, device = q.dtype, q.device
+    qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    if dtype not in _checks.TC_DTYPES or d not in _checks.TC_HEAD_DIMS or (qp | kp | vp) % 16:
+        _checks.check_tc(q, k, v)
+    od = dtype if out_dtype is None else _checks.resolve_out_dtype("fused_tc", q, out_dtype)
+    code = _DTYPE_CODE[dtype]
+    need = _LDS_NEED.get((d, code))
+    if need is None:
+        need = _lds_need((d, code), _native.lib().pa_fused_tc_lds_bytes, d, code)
+    limit = _LDS_LIMIT.get(device.index) or _lds_limit(q)
+    if not 0 <= need <= limit:
+        _checks.check_lds("fused_tc", need, limit)
+    o = torch.empty_like(q) if od is dtype else torch.empty_like(q, dtype=od)
+    _call("pa_fused_tc_fwd", "fused_tc", device, qp, kp, vp, o.data_ptr(),
+          code, _DTYPE_CODE[od], b * h, n, d, 1 if causal else 0, _stream_ptr(device))
     return o
 
 

@@ -73,6 +73,19 @@ def test_check_inputs_messages():
     chk(q, k, v)  # valid
 
 
+@pytest.mark.parametrize("at", [0, 1, 2])
+@pytest.mark.parametrize("change,match", [
+    (lambda t: t.transpose(1, 2), "contiguous"), (lambda t: t.float(), "dtype"), (lambda t: t[0], "shaped"),
+    (lambda t: t.unsqueeze(0), "shaped"), (lambda t: t[..., :32].contiguous(), "same shape"),
+    (lambda t: t.to("meta"), "same device")])
+def test_check_inputs_refuses_one_odd_input(at, change, match):
+    """The one-pass acceptance lets no single q, k or v through that the checks one by one refuse."""
+    qkv_ = list(qkv())
+    qkv_[at] = change(qkv_[at])
+    with pytest.raises(RuntimeError, match=match):
+        _checks.check_inputs(*qkv_, require_cuda=False)
+
+
 def test_head_dim_and_dtype_messages():
     q, k, v = qkv((1, 1, 64, 128))
     with pytest.raises(RuntimeError, match="head dimension"):
