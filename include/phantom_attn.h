@@ -69,12 +69,13 @@ int pa_tiled_fwd(const void* q, const void* k, const void* v, void* o, float* s,
 int pa_tiled_fwd_noalloc(const void* q, const void* k, const void* v, void* o,
                          int dtype, int64_t bh, int64_t n, int64_t d, int causal, void* stream);
 
-/* v3 fused: online softmax with fp32 arithmetic throughout: fp32 inputs on the fp32 matrix core, P
- * kept in fp32, or on larger grids on the 16-bit one with every operand in two fp16 or three bf16
- * terms (24 significant bits); fp16 inputs on the fp16 matrix core, whose products are exact, with P in two fp16
- * terms of 22 significant bits (both with errors against float64
- * below the fp32 matrix core's). fp16 calls
- * take fused_tc's launch forms, and pa_set_persistent() applies to them.
+/* v3 fused: online softmax with fp32 arithmetic, errors against float64 no larger than the fp32 matrix
+ * core's.
+ * fp32 inputs: the fp32 matrix core, or, on larger grids, the bf16 one with Q, K, V and P in three bf16
+ * terms each (24 significant bits from 2^-112 up, an absolute 2^-134 below) and the six largest term
+ * products (what is left out of a product is below 2^-25 of it).
+ * fp16 inputs: the fp16 matrix core, whose products are exact, with P in two fp16 terms of 22
+ * significant bits. These calls take fused_tc's launch forms, and pa_set_persistent() applies to them.
  * dtype: F32 or F16; out_dtype: dtype or F32; d == 64.
  * Replaces attn::launch_fused<T> (csrc/kernels/fused.cuh:106-112) and fused_forward
  * (csrc/attn_fused.cu:5-14). */

@@ -1,32 +1,33 @@
-// Fused online-softmax attention forward for fp32 inputs on the 16-bit matrix core, with fp32's
+// Fused online-softmax attention forward for fp32 inputs on the bf16 matrix core, with fp32's
 // accuracy (the `fused` entry's fp32 inputs on grids that fill the chip; fa_f32.hpp takes the rest).
 //
-// The fp32 matrix core bounds fa_f32.hpp: 64 FLOP per cycle and SIMD against the 16-bit one's 1024. Here
-// every fp32 operand (Q, K, V and P) is split into terms whose products are exact in the fp32
-// accumulator, and the small products have an accumulator of their own, so O's main chain rounds once
-// per 16 keys, not per 2. Two forms of the same block:
-//  * F16x2: x = h + l / 2^11 in fp16 (h = round(x), l = round(2^11 (x - h)): 24 bits, l normal wherever h
-//    is), three products (h h; h l, l h; what is left out is 2^-24 of a product and below). Its range:
-//    |q|, |k| <= 4096, |v| <= 255 (V is taken 2^8 larger), and no 8 dims of a V row all below 2^-20, so
-//    that what falls below the terms (2^-36 absolute) is below fp32's own rounding of the scores, and
-//    2^-24 of its row in V. Every thread looks at the values that it splits.
-//  * Bf16x3: x = h + m + l in bf16 over fp32's whole range, six products (h h; h m, m h; m m, h l, l h).
-//    Taken by a workgroup whose inputs were out of F16x2's range, as soon as Q or its first tile shows it
-//    (V x300 at 4x16x2048: 421 us, against 310 in range, timed with their host calls), else at the end of its block, which it then starts again.
-// Against float64 (2-norms; fa_f32.hpp -> F16x2, Bf16x3): 4x16x512 3.6e-7 -> 2.4e-7, 2.2e-7; 4x16x2048
-// 5.2e-7 -> 3.8e-7, 3.6e-7; 4x4x8192 8.8e-7 -> 6.4e-7, 6.4e-7; 2x4x4000 5.1e-7 -> 3.8e-7, 3.6e-7.
+// The fp32 matrix core bounds fa_f32.hpp: 64 FLOP per cycle and SIMD against the bf16 one's 1024.
+// Here every fp32 operand (Q, K, V and P) is split into three bf16 terms h + m + l, whose sum has
+// more than fp32's 24 bits (an operand below 2^-112 keeps an absolute 2^-134) and whose range is
+// fp32's, and a product takes the six term products down to 2^-18 of it (h h; h m, m h; m m, h l,
+// l h), which leaves out less than 2^-25. They are exact in the fp32 accumulator. That is
+// 1024 / 6 / 64 = 2.7x the fp32 matrix core's rate, and a smaller error: the five small products have
+// an accumulator of their own, so O's main chain rounds once per 16 keys, not per 2. Against
+// float64 (2-norms; fa_f32.hpp -> here): 4x16x512 3.6e-7 -> 2.2e-7, 4x16x2048 5.2e-7 -> 3.6e-7,
+// 4x4x8192 8.8e-7 -> 6.4e-7, causal 4x4x8000 3.8e-7 -> 2.8e-7, 2x4x4000 with Q, K x3 1.5e-6 -> 6.0e-7.
 //
 // Otherwise the fused kernels' scheme (fa_mfma.hpp): S^T = K Q^T and O^T += V^T P^T, a wave owning 32
 // queries, P^T straight from the S^T accumulator, m raised lazily. A workgroup stages 32-key tiles:
 // a thread loads 8 dims of a K and of a V row a tile ahead, splits them once for its four query waves
-// and writes the planes to LDS (two stages, one barrier per tile). KS == 2: two key groups of
+// and writes the three planes to LDS (two stages, one barrier per tile). KS == 2: two key groups of
 // four query waves walk alternate tiles and are merged at the end, which gives a CU its two waves per
 // SIMD from one workgroup.
 //
-// Measured, fa_f32.hpp -> Bf16x3 -> F16x2: 4x16x2048 601 -> 380 -> 250 us (275 TFLOP/s), 4x16x4096 2322
-// -> 1479 -> 956, causal 4x16x1024 114 -> 62 -> 47, 2x4x4000 292 -> 182 -> 122. With two waves per SIMD
-// the matrix products (24 MFMAs of 32 cycles per wave and tile, half of Bf16x3's) and the VALU (the
-// splits, the exponentials: about twice that) overlap only in part; three waves per SIMD spill (323 us).
+// Measured: 4x16x2048 601 -> 379 us (114 -> 181 TFLOP/s), 4x16x4096 2322 -> 1464 us (188), causal
+// 4x16x1024 114 -> 62 us, 2x4x4000 292 -> 185 us (177). At those sizes the six products run at
+// ~1.1 PFLOP/s of bf16 matrix work, about what a large bf16 product reaches under the card's power
+// cap; interleaving the staging with the products by scheduling groups, or a raised wave priority
+// for them, moved nothing (within 1 %), three waves per SIMD spill (146 VGPRs, 8 % slower), and
+// keeping each wave's own tiles in registers (no LDS, as fa_f32.hpp) loses 5 % to fa_f32.hpp because
+// every wave then splits its operands itself.
+// Two fp16 terms per operand (three products) are a third faster still, but hold neither a small column
+// of V beside ordinary ones nor fp32's range: below 2^-20 a value of V keeps an absolute 2^-44, a product is off by
+// up to 2^-21, and a check of every element sends a tenth of N(0, 1) heads of 2048 keys to wider terms.
 #pragma once
 
 #include "common.hpp"
@@ -91,75 +92,37 @@ __device__ __forceinline__ float join_bf3(float hi, float lo) {
   return hi + __builtin_amdgcn_fmed3f(lo, -3.4e38f, 3.4e38f);
 }
 
-// The two ways to take an operand. mfma: hi += the largest term product, lo += the small ones;
-// join: the value of the two accumulators.
-struct Bf16x3 {
-  typedef Bf3 Op;
-  typedef bf16 Elem;
-  typedef bf16x8 Vec;
-  static constexpr int PLANES = 3;
-  static constexpr float kShift = 0.f, kVScale = 1.f;
-  static constexpr bool kRanged = false;
-  static __device__ __forceinline__ Op split_input(const float (&x)[8]) { return split3_checked(x); }
-  static __device__ __forceinline__ Op split(const float (&x)[8]) { return split3(x); }
-  static __device__ __forceinline__ Vec plane(const Op& t, int i) { return i == 0 ? t.h : i == 1 ? t.m : t.l; }
-  static __device__ __forceinline__ Op from_planes(const Vec (&p)[3]) { return Op{p[0], p[1], p[2]}; }
-  static __device__ __forceinline__ void mfma(const Op& a, const Op& b, f32x16& hi, f32x16& lo) { mfma_bf3(a, b, hi, lo); }
-  static __device__ __forceinline__ float join(float hi, float lo) { return join_bf3(hi, lo); }
-};
-struct F16x2 {
-  struct Op {
-    f16x8 h, l;
-  };
-  typedef f16 Elem;
-  typedef f16x8 Vec;
-  static constexpr int PLANES = 2;
-  static constexpr float kShift = 15.f;     // P <= 2^15
-  static constexpr float kVScale = 256.f;
-  static constexpr bool kRanged = true;
-  static __device__ __forceinline__ Op split(const float (&x)[8]) {
-    Op t;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t.h[j] = (f16)x[j];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t.l[j] = (f16)((x[j] - (float)t.h[j]) * 2048.f);
-    return t;
-  }
-  static __device__ __forceinline__ Op split_input(const float (&x)[8]) { return split(x); }
-  static __device__ __forceinline__ Vec plane(const Op& t, int i) { return i == 0 ? t.h : t.l; }
-  static __device__ __forceinline__ Op from_planes(const Vec (&p)[2]) { return Op{p[0], p[1]}; }
-  static __device__ __forceinline__ void mfma(const Op& a, const Op& b, f32x16& hi, f32x16& lo) {
-    lo = mfma32x32x16(a.l, b.h, lo);
-    lo = mfma32x32x16(a.h, b.l, lo);
-    hi = mfma32x32x16(a.h, b.h, hi);
-  }
-  static __device__ __forceinline__ float join(float hi, float lo) { return fmaf(lo, 1.f / 2048.f, hi); }
-};
-
-// One block of queries of one head. False (F16x2 only): an input was out of its range, and nothing
-// was stored.
-template <typename TM, int D, int NQ, int KS>
-__device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, const float* __restrict__ K,
-                                                const float* __restrict__ V, float* __restrict__ O, int N, int bh, int qb,
-                                                float scale_log2, int causal, unsigned char* k_lds0, unsigned char* v_lds0,
-                                                unsigned char* k_lds1, unsigned char* v_lds1, float* red_ml, int* red_bad) {
-  typedef typename TM::Op Op;
-  typedef typename TM::Vec Vec;
-  constexpr int PLANES = TM::PLANES;
+template <int D, int NQ, int KS>
+__global__ void __launch_bounds__(NQ * KS * kWave)
+__attribute__((amdgpu_waves_per_eu(2)))
+fa_f32x3_fwd(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+             float* __restrict__ O, int N, int num_qblocks, int total_blocks, float scale_log2, int causal) {
   constexpr int BM = NQ * 32, BN = 32;
-  constexpr int CR = D / 8, RB = D * 2, PLANE = BN * RB, MAT = PLANES * PLANE;   // term planes of a tile
+  constexpr int CR = D / 8, RB = D * 2, PLANE = BN * RB, MAT = 3 * PLANE;   // bf16 planes of a tile
   constexpr int STEPS = D / 16, NDB = D / 32;
   constexpr int CPT = BN * CR / (NQ * kWave);   // 8-dim chunks of K and of V per thread and tile
   // m is set to a row's max plus kLazyLog2 and raised again only when the max has passed it, so
-  // P = 2^(s c - m) stays at most 1 (P V cannot overflow where V does not), F16x2: 2^15.
+  // P = 2^(s c - m) stays at most 1, a row's largest between 2^-8 and 1: no single product P V overflows
+  // where V does not, and a row's sum of them later than with m at the max.
   constexpr float kLazyLog2 = 8.f;
-  constexpr float kQKMax = 4096.f, kVMax = 255.f, kVLow = 0x1p-20f;   // F16x2's range
   static_assert(D == 64 && CPT * NQ * kWave == BN * CR, "whole chunks per thread");
+  __shared__ __attribute__((aligned(1024))) unsigned char k_lds0[KS * MAT], v_lds0[KS * MAT], k_lds1[KS * MAT], v_lds1[KS * MAT];
+  __shared__ float red_ml[KS > 1 ? (KS - 1) * NQ * 2 * kWave : 1];
   const int g = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / (NQ * kWave));   // key group
   const int tid = (int)threadIdx.x % (NQ * kWave), lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lq = lane % 32, hi = lane / 32;
 
+  int bh, qb;
+  if (causal) {   // the longest blocks of every head first; with B*H a multiple of 8 a head keeps its XCD
+    const int heads = total_blocks / num_qblocks;
+    qb = num_qblocks - 1 - (int)blockIdx.x / heads;
+    bh = (int)blockIdx.x % heads;
+  } else {
+    const int blk = xcd_remap(blockIdx.x, total_blocks);
+    bh = blk / num_qblocks;
+    qb = blk % num_qblocks;
+  }
   const int q0 = qb * BM, q0w = q0 + wave * 32, qrow = q0w + lq;
   const size_t base = (size_t)bh * N * D;
   const uint32_t head_bytes = (uint32_t)((size_t)N * D * 4);
@@ -175,21 +138,12 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
   };
 
   // Q^T operand terms: dims 16 kk + 8 hi .. + 7 of row qrow (rows past N read as zero).
-  Op qf[STEPS];
-  float qk_max = 0.f, v_max = 0.f;   // F16x2: what its range check looks at
-  bool v_low = false;
-  auto abs_max = [](const float (&x)[8]) __attribute__((always_inline)) {
-    float m = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(x[j]));
-    return m;
-  };
+  Bf3 qf[STEPS];
 #pragma unroll
   for (int kk = 0; kk < STEPS; ++kk) {
     float x[8];
     load8(q_rs, (uint32_t)((qrow * D + 16 * kk + 8 * hi) * 4), x);
-    if constexpr (TM::kRanged) qk_max = fmaxf(qk_max, abs_max(x));
-    qf[kk] = TM::split_input(x);
+    qf[kk] = split3_checked(x);
   }
 
   // Staging: a thread carries CPT chunks of its key group's K and V tiles, global to registers one
@@ -215,20 +169,14 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
   auto stage = [&](unsigned char* ks, unsigned char* vs) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-      if constexpr (TM::kRanged) {
-        qk_max = fmaxf(qk_max, abs_max(kx[i]));
-        const float m = abs_max(vx[i]);
-        v_max = fmaxf(v_max, m);
-        v_low |= m < kVLow && m > 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vx[i][j] *= TM::kVScale;
-      }
-      const Op a = TM::split_input(kx[i]), b = TM::split_input(vx[i]);
-#pragma unroll
-      for (int pl = 0; pl < PLANES; ++pl) {
-        *reinterpret_cast<Vec*>(ks + pl * PLANE + k_dst[i]) = TM::plane(a, pl);
-        *reinterpret_cast<Vec*>(vs + pl * PLANE + v_dst[i]) = TM::plane(b, pl);
-      }
+      const Bf3 a = split3_checked(kx[i]);
+      *reinterpret_cast<bf16x8*>(ks + k_dst[i]) = a.h;
+      *reinterpret_cast<bf16x8*>(ks + PLANE + k_dst[i]) = a.m;
+      *reinterpret_cast<bf16x8*>(ks + 2 * PLANE + k_dst[i]) = a.l;
+      const Bf3 b = split3_checked(vx[i]);
+      *reinterpret_cast<bf16x8*>(vs + v_dst[i]) = b.h;
+      *reinterpret_cast<bf16x8*>(vs + PLANE + v_dst[i]) = b.m;
+      *reinterpret_cast<bf16x8*>(vs + 2 * PLANE + v_dst[i]) = b.l;
     }
   };
 
@@ -259,14 +207,15 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
     f32x16 sh = f32x16{}, sl = f32x16{};
 #pragma unroll
     for (int kk = 0; kk < STEPS; ++kk) {
-      Vec a[PLANES];
-#pragma unroll
-      for (int pl = 0; pl < PLANES; ++pl) a[pl] = *reinterpret_cast<const Vec*>(ks + pl * PLANE + k_addr[kk]);
-      TM::mfma(TM::from_planes(a), qf[kk], sh, sl);
+      Bf3 a;
+      a.h = *reinterpret_cast<const bf16x8*>(ks + k_addr[kk]);
+      a.m = *reinterpret_cast<const bf16x8*>(ks + PLANE + k_addr[kk]);
+      a.l = *reinterpret_cast<const bf16x8*>(ks + 2 * PLANE + k_addr[kk]);
+      mfma_bf3(a, qf[kk], sh, sl);
     }
     float s[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = TM::join(sh[r], sl[r]);
+    for (int r = 0; r < 16; ++r) s[r] = join_bf3(sh[r], sl[r]);
     if (t >= clean_tiles) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -285,7 +234,7 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
 #pragma unroll
       for (int db = 0; db < NDB; ++db) oh[db] *= alpha, ol[db] *= alpha;
     }
-    const float nm = m_run == -INFINITY ? 0.f : TM::kShift - m_run;   // no visible key so far: P = 0
+    const float nm = m_run == -INFINITY ? 0.f : -m_run;   // no visible key so far: P = 0
     float p[2][8];
     float sum[2] = {0.f, 0.f};                            // the tile's sum first, then one add to l
 #pragma unroll
@@ -296,32 +245,20 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
     l_run += sum[0] + sum[1];
 #pragma unroll
     for (int k2 = 0; k2 < 2; ++k2) {
-      const Op pf = TM::split(p[k2]);
+      const Bf3 pf = split3(p[k2]);
 #pragma unroll
       for (int db = 0; db < NDB; ++db) {
-        Vec a[PLANES];
+        bf16x8 a[3];
 #pragma unroll
-        for (int pl = 0; pl < PLANES; ++pl) {
+        for (int pl = 0; pl < 3; ++pl) {
           const unsigned char* p0 = vs + pl * PLANE + k2 * 16 * RB + v_addr[db];
           const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0));
           const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0 + 8 * RB));
-          a[pl] = __builtin_bit_cast(Vec, i16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]});
+          a[pl] = __builtin_bit_cast(bf16x8, i16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]});
         }
-        TM::mfma(TM::from_planes(a), pf, oh[db], ol[db]);
+        mfma_bf3(Bf3{a[0], a[1], a[2]}, pf, oh[db], ol[db]);
       }
     }
-  };
-
-  // F16x2: whether a value that some thread has split so far was out of range (all threads get the
-  // same answer). (A NaN is in range: it goes through the terms to where it belongs.)
-  auto out_of_range = [&]() __attribute__((always_inline)) {
-    const bool bad = __builtin_amdgcn_ballot_w64(qk_max > kQKMax || v_max > kVMax || v_low) != 0;
-    if (lane == 0) red_bad[(int)threadIdx.x / kWave] = bad;
-    __syncthreads();
-    int any = 0;
-#pragma unroll
-    for (int w = 0; w < NQ * KS; ++w) any |= red_bad[w];
-    return __builtin_amdgcn_readfirstlane(any) != 0;
   };
 
   // Tile j + 1 is staged, and tile j + 2 loaded, before tile j's products; one barrier per tile
@@ -329,14 +266,7 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
   gload(0);
   stage(k_lds0, v_lds0);
   gload(1);
-  if constexpr (TM::kRanged) {   // Q and the first tile: inputs of another scale show here
-    if (out_of_range()) {
-      __syncthreads();
-      return false;
-    }
-  } else {
-    __syncthreads();
-  }
+  __syncthreads();
   for (int j = 0; j < nit; j += 2) {
     stage(k_lds1, v_lds1);
     gload(j + 2);
@@ -350,22 +280,15 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
     }
   }
 
-  if constexpr (TM::kRanged) {
-    if (out_of_range()) {
-      __syncthreads();   // (Bf16x3 writes what slower waves may still read)
-      return false;
-    }
-  }
-
   f32x16 o[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[db][r] = TM::join(oh[db][r], ol[db][r]);
+    for (int r = 0; r < 16; ++r) o[db][r] = join_bf3(oh[db][r], ol[db][r]);
   float l = half_sum(l_run);
   // Key groups: group 0 merges the others' (m, l, O), handed over through the free stages.
   if constexpr (KS > 1) {
-    static_assert(KS == 2 && NQ * NDB * 16 * kWave * 4 <= 2 * KS * 3 * PLANE, "merge through two stages");
+    static_assert(KS == 2 && NQ * NDB * 16 * kWave * 4 <= 2 * KS * MAT, "merge through two stages");
     float* red_o = reinterpret_cast<float*>(wave < NQ / 2 ? k_lds0 : v_lds0) + (wave % (NQ / 2)) * (NDB * 16 * kWave);
     float* ml = red_ml + wave * 2 * kWave;
     if (g == 1) {
@@ -377,7 +300,7 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
       ml[kWave + lane] = l;
     }
     __syncthreads();
-    if (g == 1) return true;
+    if (g == 1) return;
     const float m1 = ml[lane], l1 = ml[kWave + lane];
     const float m = fmaxf(m_run, m1);
     const float sc0 = m_run == -INFINITY ? 0.f : exp2_fast(m_run - m);
@@ -389,7 +312,7 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
       for (int r = 0; r < 16; ++r) o[db][r] = sc0 * o[db][r] + sc1 * red_o[(db * 16 + r) * kWave + lane];
   }
   if (qrow < N) {
-    const float inv = 1.f / (TM::kVScale * l);
+    const float inv = 1.f / l;
     float* orow = O + base + (size_t)qrow * D;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
@@ -401,32 +324,6 @@ __device__ __forceinline__ bool f32_terms_block(const float* __restrict__ Q, con
         *reinterpret_cast<f32x4*>(orow + db * 32 + g4 * 8 + hi * 4) = w;
       }
   }
-  return true;
-}
-
-template <int D, int NQ, int KS>
-__global__ void __launch_bounds__(NQ * KS * kWave)
-__attribute__((amdgpu_waves_per_eu(2)))
-fa_f32_terms_fwd(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
-             float* __restrict__ O, int N, int num_qblocks, int total_blocks, float scale_log2, int causal) {
-  constexpr int MAT = 3 * 32 * D * 2;   // the planes of a 32-key tile in the larger form
-  __shared__ __attribute__((aligned(1024))) unsigned char k_lds0[KS * MAT], v_lds0[KS * MAT], k_lds1[KS * MAT], v_lds1[KS * MAT];
-  __shared__ float red_ml[KS > 1 ? (KS - 1) * NQ * 2 * kWave : 1];
-  __shared__ int red_bad[NQ * KS];
-  int bh, qb;
-  if (causal) {   // the longest blocks of every head first; with B*H a multiple of 8 a head keeps its XCD
-    const int heads = total_blocks / num_qblocks;
-    qb = num_qblocks - 1 - (int)blockIdx.x / heads;
-    bh = (int)blockIdx.x % heads;
-  } else {
-    const int blk = xcd_remap(blockIdx.x, total_blocks);
-    bh = blk / num_qblocks;
-    qb = blk % num_qblocks;
-  }
-  if (!f32_terms_block<F16x2, D, NQ, KS>(Q, K, V, O, N, bh, qb, scale_log2, causal, k_lds0, v_lds0, k_lds1, v_lds1, red_ml,
-                                         red_bad))
-    f32_terms_block<Bf16x3, D, NQ, KS>(Q, K, V, O, N, bh, qb, scale_log2, causal, k_lds0, v_lds0, k_lds1, v_lds1, red_ml,
-                                       red_bad);
 }
 
 }  // namespace pa

@@ -20,7 +20,7 @@
 
 #include "phantom_attn.h"
 #include "kernels/fa_f32.hpp"
-#include "kernels/fa_f32_terms.hpp"
+#include "kernels/fa_f32x3.hpp"
 #include "kernels/fa_mfma.hpp"
 #include "kernels/unfused.hpp"
 #include "launch_model.hpp"
@@ -360,36 +360,36 @@ const MfmaEntry* find_tuned(int dtype, int out_dtype, int64_t d, int br, int bc,
 }
 
 // ------------------------------------------------------------------ fused, fp32 arithmetic
-// fp32 inputs. fa_f32_fwd (fp32 matrix core): 32 query rows per workgroup, keys split over kF32KS
-// waves. fa_f32_terms_fwd (16-bit matrix core, operands split into terms): 128 query rows per workgroup, in
-// one key group of 4 waves or two of them.
+// fp32 inputs, three kernels. fa_f32_fwd (fp32 matrix core): 32 query rows per workgroup, keys split
+// over kF32KS waves. fa_f32x3_fwd (bf16 matrix core, three-term operands): 128 query rows per
+// workgroup, in one key group of 4 waves or two of them.
 constexpr int kF32KS = 4;
-// The terms have 5x the fp32 matrix core's rate but a quarter of its workgroups (four waves share a
-// staged tile), so they are taken where those would put a second workgroup on many CUs (short rows, where
-// the staging is a larger part: on every second CU), and a row has more than one 32-key tile. Measured,
-// fa_f32_fwd -> fa_f32_terms_fwd in us (128-query blocks in brackets): 64x256 (128) 17.3 -> 15.0, 16x1024
-// (128) 48.6 -> 34.2, 8x2048 (128) 83.5 -> 58.6, causal 63.2 -> 57.9, causal 3x5000 (120) 157 -> 130,
-// 150x96 10.6 -> 9.2, 200x64 9.6 -> 7.7; below the line 32x256 (64) 11.1 -> 13.6, 8x1024 (64) 27.1 ->
-// 32.3, 4x2048 (64) 50.1 -> 57.3, 100x128 11.0 -> 10.5, causal 10.6 -> 11.2; rows of one tile gain
-// nothing at any count (1000x32 13.0 -> 12.9).
-bool use_f32_terms(int64_t n, int64_t blocks) { return n > 32 && blocks > (n <= 128 ? 128 : 96); }
+// The bf16 terms have 2.7x the fp32 matrix core's rate but a quarter of its workgroups (four waves
+// share a staged tile; with their own tiles the splitting costs what the rate gains), so they are
+// taken where the 128-query blocks outnumber half the CUs (short rows: 160, the staging is a larger
+// part of them) and a row has more than one 32-key tile. Measured, fa_f32_fwd -> fa_f32x3_fwd in us:
+// 64 heads x 256 (128 blocks) 15.2 -> 15.7, 16x1000 (128) 44.7 -> 43.1, causal 3x5000 (120) 153 ->
+// 181, 150x96 9.0 -> 9.6; above the line 96x256 (192) 22.8 -> 16.2, 9x2048 (144) 118 -> 79, causal
+// 5x4096 (160) 166 -> 150, 200x64 8.3 -> 7.8, 400x33 14.3 -> 10.5; rows of one tile lose at any
+// count (1000x32 10.5 -> 13.0).
+bool use_bf16_terms(int64_t n, int64_t blocks) { return n > 32 && blocks > (n <= 128 ? 160 : 128); }
 // Two key groups (8 waves, one workgroup per CU) where one group would leave the CUs a workgroup of
-// 4 waves or less to end on: up to one block per CU, and causal, whose blocks differ in length, two. One
-// group -> two, us: 96x256 (192) 15.9 -> 15.6, 64x512 (256) 26.8 -> 24.0, 8x4096 (256) 152 -> 120, causal
-// 40x1024 (320) 44.4 -> 35.3, 12x4096 (384) 154 -> 114, 32x2048 (512) 84.8 -> 72.6, 64x1024 (512) 47.1 ->
-// 45.6; beyond: 80x512 (320) 35.5 -> 41.3, 40x1024 (320) 60.9 -> 66.7, 12x4096 (384) 222 -> 222, causal
-// 80x1024 (640) 52.3 -> 62.6; short rows 160x128 11.0 -> 12.3.
-bool use_f32_terms_key_groups(int64_t n, int64_t blocks, int causal) {
-  return n > 128 && blocks <= (causal ? 2 : 1) * kCUs;
+// 4 waves or less to end on: up to one block per CU, and up to two for rows of 1024 keys or more.
+// One group -> two, us: 96x256 (192) 18.5 -> 16.2, 64x512 (256) 32.7 -> 28.7, causal 7x4096 (224)
+// 216 -> 150, 24x2048 (384) 176 -> 168, causal 40x1024 (320) 60.6 -> 45.9, causal 64x1024 (512)
+// 67 -> 62, 16x4096 (512) 378 -> 360; beyond: causal 128x1024 (1024) 112 -> 123, 100x512 (400) 50.3 ->
+// 51.8, 324x128 (324) 17.9 -> 22.5.
+bool use_f32x3_key_groups(int64_t n, int64_t blocks) {
+  return (n > 128 && blocks <= kCUs) || (n >= 1024 && blocks <= 2 * kCUs);
 }
 
 hipError_t launch_f32(const void* q, const void* k, const void* v, void* o, int bh, int n, int causal,
                       hipStream_t stream) {
   const long long blocks = (long long)((n + 127) / 128) * bh;
   if (blocks > INT_MAX) return hipErrorInvalidConfiguration;
-  if (use_f32_terms(n, blocks)) {
-    const bool groups = use_f32_terms_key_groups(n, blocks, causal);
-    auto kernel = groups ? pa::fa_f32_terms_fwd<64, 4, 2> : pa::fa_f32_terms_fwd<64, 4, 1>;
+  if (use_bf16_terms(n, blocks)) {
+    const bool groups = use_f32x3_key_groups(n, blocks);
+    auto kernel = groups ? pa::fa_f32x3_fwd<64, 4, 2> : pa::fa_f32x3_fwd<64, 4, 1>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(4 * (groups ? 2 : 1) * pa::kWave), 0, stream,
                        static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                        static_cast<float*>(o), n, (n + 127) / 128, (int)blocks, scale_log2_for(64), causal);

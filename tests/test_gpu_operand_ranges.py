@@ -1,0 +1,73 @@
+"""Operands of unusual scale through the entry points whose arithmetic is fp32 (fused, tiled, naive).
+
+fp32 arithmetic holds every weight and value to 24 bits of itself, whatever stands beside it: a small
+column of V, a small probability, a value near the largest float, an infinity. The kernels that take
+operands in 16-bit terms or sum before they normalise are held to that here.
+"""
+import math
+
+import pytest
+import torch
+
+import cuda_attn
+from cuda_attn import _native
+from cuda_attn.workloads import make_qkv
+
+pytestmark = pytest.mark.gpu
+
+F32, F16 = torch.float32, torch.float16
+INF = float("inf")
+# Grids of each form of fused with fp32 inputs: the fp32 matrix core, two key groups, one key group.
+FUSED_F32_GRIDS = [(3, 300), (60, 300), (300, 300), (8, 4096), (80, 1024)]
+
+
+def reference64(q, k, v, causal=False):
+    """float64 softmax(QK^T/sqrt(d))V of the visible keys (a head at a time; V may hold infinities)."""
+    b, h, n, d = q.shape
+    out = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+    for i in range(b):
+        for j in range(h):
+            s = torch.matmul(q[i, j].double(), k[i, j].double().t().contiguous()) / math.sqrt(d)
+            if causal:
+                s.masked_fill_(torch.ones_like(s, dtype=torch.bool).triu(1), -INF)
+            out[i, j] = torch.matmul(torch.softmax(s, -1), v[i, j].double())
+    return out
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("large", [False, True])
+@pytest.mark.parametrize("bh,n", FUSED_F32_GRIDS)
+def test_fused_fp32_column_scales(bh, n, large, causal):
+    """Columns of V of very different scales beside each other (and on both sides of 2^-20): an output
+    column depends on its own column of V alone, so its relative error does not depend on the scale.
+    4e-6 in the 2-norm per head and column (fp32 sums are seen 2e-7 to 1.2e-6 off)."""
+    q, k, v = make_qkv(1, bh, n, 64, F32, seed=17, device="cuda")
+    scale = torch.ones(64, device="cuda")
+    scale[8:16] = torch.tensor([1.0, 2.0 ** -17, 2.0 ** -20, 2.0 ** -23, 1e-8, 1e-10, 1e-12, 1e-14])
+    scale[20], scale[30] = 1e-20, 1e-30
+    if large:
+        scale[21], scale[40] = 1e4, 1e25
+    v = v * scale
+    heads = list(range(0, bh, max(1, bh // 4)))
+    out = cuda_attn.fused(q, k, v, causal)[:, heads].double()
+    ref = reference64(q[:, heads], k[:, heads], v[:, heads], causal)
+    err = torch.linalg.vector_norm(out - ref, dim=2) / torch.linalg.vector_norm(ref, dim=2)
+    assert err.max().item() <= 4e-6
+
+
+@pytest.mark.parametrize("bh,n", FUSED_F32_GRIDS)
+def test_fused_fp32_single_products(bh, n):
+    """Scores of a single product each (one nonzero dim in Q): no sum averages the operands' roundings.
+    Three roundings of fp32 of a score in the log2 domain (|x| <= X) put a probability off by at most
+    ln 2 * 3 * 2^-24 X, an output by twice that of the largest |V|, and 2e-6 for the other steps."""
+    q, k, v = make_qkv(1, bh, n, 64, F32, seed=23, device="cuda")
+    q[..., :11] = 0
+    q[..., 12:] = 0
+    q[..., 11] *= 30
+    k[..., 11] *= 4
+    heads = list(range(0, bh, max(1, bh // 4)))
+    out = cuda_attn.fused(q, k, v)[:, heads].double()
+    ref = reference64(q[:, heads], k[:, heads], v[:, heads])
+    x = (q[..., 11].abs() / 8 * 1.4427)[:, heads].unsqueeze(-1) * k[..., 11].abs()[:, heads].amax(-1)[..., None, None]
+    bound = (2 * math.log(2) * 3 * 2.0 ** -24 * x + 2e-6) * v.abs().max()
+    assert bool(((out - ref).abs() <= bound).all())

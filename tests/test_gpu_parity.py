@@ -502,8 +502,8 @@ def test_fused_fp16_infinite_value_stays_infinite():
     assert torch.equal(out[keep], want[keep])
 
 
-# fused with fp32 inputs: the fp32 matrix core on small grids, operands split into 16-bit terms on larger
-# ones (one or two key groups; two fp16 terms, or three bf16 terms where a value is out of their range).
+# fused with fp32 inputs: the fp32 matrix core on small grids, operands split into three bf16 terms on larger
+# ones (one or two key groups).
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("bh,n", [(128, 128), (161, 33), (161, 64), (161, 65), (162, 128), (129, 129), (300, 96),
                                   (260, 160), (64, 257), (70, 255), (17, 1000), (33, 1024), (65, 1023), (9, 2049),
@@ -521,9 +521,8 @@ def test_fused_fp32_forms(bh, n, causal):
 @pytest.mark.parametrize("scale", [(1, 1, 1e-8), (1, 1, 1e-3), (1, 1, 60), (1, 1, 1e4), (1, 1, 1e30), (1e-4, 1, 1),
                                    (1e-3, 900, 1), (1e-6, 1e5, 1), (1e5, 1e-6, 1), (1e-20, 1e20, 1e-20)])
 def test_fused_fp32_operand_scales(bh, n, scale):
-    """q, k and v at scales inside, across (60: some values past 255, 900: past 4096) and outside the range
-    of the fp16 terms, and one block's rows outside it alone: against float64, 4e-6 in the 2-norm per head
-    (fp32 sums are seen 2e-7 to 1.2e-6 off)."""
+    """q, k and v at scales inside, across and outside fp16's range, and one block's rows at another scale
+    than the rest: against float64, 4e-6 in the 2-norm per head (fp32 sums are seen 2e-7 to 1.2e-6 off)."""
     q, k, v = gpu_qkv(1, bh, n, 64, torch.float32, seed=13)
     q, k, v = q * scale[0], k * scale[1], v * scale[2]
     q[0, 1, 130:140] *= 2.0 ** 14
@@ -552,7 +551,6 @@ def test_fused_fp32_range(bh, n):
     want = cuda_attn.fused(q, k, torch.where(v.isinf(), torch.zeros_like(v), v))
     assert (out[0, 1, :, 3] == float("inf")).all()
     keep = torch.arange(64, device="cuda") != 3
-    # (The head with the infinity takes the wider terms, the one without may not: both within F32_BAR.)
     assert max_err(out[0, 1][:, keep], want[0, 1][:, keep]) <= 2 * F32_BAR
     rest = torch.arange(n, device="cuda") != 5
     s = (q[0, 2].double() @ k[0, 2][rest].double().t()) / 8.0
