@@ -226,10 +226,12 @@ fa_f32x3_fwd(const float* __restrict__ Q, const float* __restrict__ K, const flo
     float mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    // (A row is raised for its own max alone: causal rows' bits do not depend on later tokens.)
     const float m_new = fmaxf(m_run, fmaf(half_max(mx), scale_log2, kLazyLog2));
-    if (__builtin_amdgcn_ballot_w64(m_new > m_run + kLazyLog2) != 0) {
-      const float alpha = m_new > m_run ? exp2_fast(m_run - m_new) : 1.f;   // m_run = -inf -> 0
-      m_run = m_new;
+    const bool raise = m_new > m_run + kLazyLog2;
+    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+      const float alpha = raise ? exp2_fast(m_run - m_new) : 1.f;   // m_run = -inf -> 0
+      m_run = raise ? m_new : m_run;
       l_run *= alpha;
 #pragma unroll
       for (int db = 0; db < NDB; ++db) oh[db] *= alpha, ol[db] *= alpha;

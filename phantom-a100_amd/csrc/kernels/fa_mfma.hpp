@@ -425,16 +425,18 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
 
   // Row max of a masked tile. `rescale` is set, wave-uniform, when some row's max exceeds its
   // reference max m_run by more than 2^kLazyLog2; then every row whose max grew takes it as its
-  // new m_run. Returns alpha = 2^(m_old - m_new): 0 on a row's first visible tile, exactly 1
-  // where m_run is kept.
+  // new m_run (TERMS == 2: only the rows past their own threshold do, so that causal rows' bits do
+  // not depend on later tokens). Returns alpha = 2^(m_old - m_new): 0 on a row's first visible tile,
+  // exactly 1 where m_run is kept.
   auto update_max = [&](const f32x16 (&s)[NKB], bool& rescale) -> float {
     float mx = -INFINITY;
 #pragma unroll
     for (int b = 0; b < NKB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[b][r]);
-    const float m_new = fmaxf(m_run, half_max(mx) * scale_log2);
-    rescale = __builtin_amdgcn_ballot_w64(m_new > m_run + kLazyLog2) != 0;
+    float m_new = fmaxf(m_run, half_max(mx) * scale_log2);
+    if constexpr (TERMS == 2) m_new = m_new > m_run + kLazyLog2 ? m_new : m_run;
+    rescale = __builtin_amdgcn_ballot_w64(TERMS == 2 ? m_new > m_run : m_new > m_run + kLazyLog2) != 0;
     const bool upd = rescale && m_new > m_run;
     const float alpha = upd ? exp2_fast(m_run - m_new) : 1.f;  // m_run = -inf -> 0
     m_run = upd ? m_new : m_run;

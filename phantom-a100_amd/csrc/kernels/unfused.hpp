@@ -435,10 +435,12 @@ tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __rest
     for (int i = 0; i < NG; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) mx = fmaxf(mx, x[i][e]);
+    // (A row is raised for its own max alone: causal rows' bits do not depend on later tokens.)
     const float m_new = fmaxf(m_run, half_max(mx) * scale_log2);
-    if (__builtin_amdgcn_ballot_w64(m_new > m_run + kLazyLog2) != 0) {
-      const float alpha = m_new > m_run ? exp2_fast(m_run - m_new) : 1.f;   // m_run = -inf -> 0
-      m_run = m_new;
+    const bool raise = m_new > m_run + kLazyLog2;
+    if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+      const float alpha = raise ? exp2_fast(m_run - m_new) : 1.f;   // m_run = -inf -> 0
+      m_run = raise ? m_new : m_run;
       l_run *= alpha;
 #pragma unroll
       for (int db = 0; db < NDB; ++db) o[db] *= alpha;

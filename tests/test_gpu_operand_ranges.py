@@ -55,6 +55,21 @@ def test_fused_fp32_column_scales(bh, n, large, causal):
     assert err.max().item() <= 4e-6
 
 
+@pytest.mark.parametrize("name,dtype,bh,n", [("fused", F32, *g) for g in FUSED_F32_GRIDS] +
+                         [("fused", F16, *g) for g in ((2, 300), (300, 320), (300, 200), (140, 1000), (300, 40))] +
+                         [("tiled", dt, *g) for dt in (F32, F16) for g in ((2, 300), (64, 515))])
+def test_causal_rows_do_not_see_later_tokens(name, dtype, bh, n):
+    """Causal rows keep their bits when only later tokens change, to scores and values of another scale."""
+    q, k, v = make_qkv(1, bh, n, 64, dtype, seed=19, device="cuda")
+    out = getattr(cuda_attn, name)(q, k, v, True)
+    for j in (n // 2 + 5, n - 3):
+        k2, v2 = k.clone(), v.clone()
+        k2[:, :, j:] *= 500
+        v2[:, :, j:] *= 1e9 if dtype == F32 else 1e3
+        same = torch.equal(getattr(cuda_attn, name)(q, k2, v2, True)[:, :, :j], out[:, :, :j])
+        assert same, j
+
+
 @pytest.mark.parametrize("bh,n", FUSED_F32_GRIDS)
 def test_fused_fp32_single_products(bh, n):
     """Scores of a single product each (one nonzero dim in Q): no sum averages the operands' roundings.
