@@ -74,8 +74,9 @@ int pa_tiled_fwd_noalloc(const void* q, const void* k, const void* v, void* o,
  * fp32 inputs: the fp32 matrix core, or, on larger grids, the bf16 one with Q, K, V and P in three bf16
  * terms each (24 significant bits from 2^-112 up, an absolute 2^-134 below) and the six largest term
  * products (what is left out of a product is below 2^-25 of it).
- * fp16 inputs: the fp16 matrix core, whose products are exact, with P in two fp16 terms of 22
- * significant bits. These calls take fused_tc's launch forms, and pa_set_persistent() applies to them.
+ * fp16 inputs: the fp16 matrix core, whose products are exact, with P in two fp16 terms (22
+ * significant bits of a weight down to 2^-21 of its row's largest, an absolute 2^-43 of that below, which
+ * fp16 output does not show). These calls take fused_tc's launch forms, and pa_set_persistent() applies to them.
  * dtype: F32 or F16; out_dtype: dtype or F32; d == 64.
  * Replaces attn::launch_fused<T> (csrc/kernels/fused.cuh:106-112) and fused_forward
  * (csrc/attn_fused.cu:5-14). */

@@ -145,8 +145,10 @@ constexpr int mfma_min_waves() {
 }
 
 // TERMS == 2 (fp16, the row-max forms; the `fused` entry's fp16 calls, which promise fp32 arithmetic):
-// P is not rounded to fp16 but taken as two fp16 terms, hi = round(P') and lo = round(P' - hi), 22
-// significant bits, and both go through P.V and the row sum. Products of fp16 values are exact in
+// P is not rounded to fp16 but taken as two fp16 terms, hi = round(P') and lo = round(2^11 (P' - hi)),
+// and both go through P.V and the row sum: 22 significant bits of every weight down to 2^-21 of the row's
+// largest, an absolute 2^-43 of that below (lo unscaled, as short to compute, would be subnormal from
+// 2^-10 of the reference: a weight of 2^-28 4e-3 off). Products of fp16 values are exact in
 // the fp32 accumulator, and so is Q K^T, so the result has fp32 arithmetic's error: against float64,
 // fp32 output, B x H x N = 1x42x128 / 4x16x2048 / 4x4x8192 / causal 4x4x8000 / 2x4x4000 with Q, K x3,
 // the fp32 matrix core's kernel was 3.0e-7 / 5.2e-7 / 8.8e-7 / 3.8e-7 / 1.5e-6 off and this one
@@ -156,7 +158,7 @@ constexpr int mfma_min_waves() {
 // MFMAs of 32x32x16 and 8 of 16x16x32 per 64-key tile against ~5 VALU instructions a score), where
 // the fp32 matrix core has 1/16 of the rate. Time, fp32 matrix core -> this: 4x16x4096 2347 -> 469 us
 // (117 -> 586 TFLOP/s), 8x16x1024 315 -> 63 us, causal 4x16x1024 108 -> 23 us, 1x42x128 6.0 -> 5.0.
-// The interleave (8 and 4 VALU instructions per MFMA) is within 2 % for 4-8 and 3-6.
+// The interleave (8 and 4 VALU instructions per MFMA) is within 2 % for 4-12 and 3-6.
 // CHECK (fp16, two stages, no key split, not the causal form): the lazy rescale is triggered by a
 // check on the computed P' (as the bf16 kernels always do) instead of the row max of S before the
 // exponentials; see the branch below.
@@ -171,8 +173,9 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
   typedef MfmaLds<D, BN, STAGES> L;
   constexpr float kLazyLog2 = 8.f;       // P stays below 2^kLazyLog2 between rescales
   // TERMS == 2: P is taken 2^7 larger (its reference m - 7, in numerator and denominator alike), so
-  // P' <= 2^15 < 65504 and its lo term stays a normal fp16 down to P = 2^-10.
-  constexpr float kTermShift = TERMS == 2 ? 7.f : 0.f;
+  // P' <= 2^15 < 65504, and its lo term 2^11 larger still. (Both in the exponent's argument would
+  // round it twice as coarsely: error with fp32 output 1.7e-7 -> 3.4e-7 at 42x128.)
+  constexpr float kTermShift = TERMS == 2 ? 7.f : 0.f, kLoScale = 2048.f;
   constexpr int NW = BM / 32;
   constexpr int THREADS = NW * kWave;
   constexpr int QK_STEPS = D / 16;       // MFMA k-steps over the head dim
@@ -355,7 +358,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] = __builtin_isfinite(o[db][r]) ? o[db][r] + o_lo[db][r] : o[db][r];
+        for (int r = 0; r < 16; ++r) o[db][r] = __builtin_isfinite(o[db][r]) ? fmaf(o_lo[db][r], 1.f / kLoScale, o[db][r]) : o[db][r];
   };
 
   const int kv_end = causal ? min(N, q0 + BM) : N;
@@ -456,10 +459,13 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
   auto row_sum = [&](const V8 (&pf)[PF]) {
     if constexpr (TERMS == 2) {
       // A tile's sum first, then one fp32 add to l (instead of 2 PV_STEPS roundings at l's size).
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
+      f32x4 t = {0.f, 0.f, 0.f, 0.f}, tl = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < PF; ++i) t = mfma16x16x32(ones, pf[PF - 1 - i], t);
-      lacc[0] += t[0];
+      for (int i = 0; i < PV_STEPS; ++i) {
+        t = mfma16x16x32(ones, pf[i], t);
+        tl = mfma16x16x32(ones, pf[PV_STEPS + i], tl);
+      }
+      lacc[0] += fmaf(tl[0], 1.f / kLoScale, t[0]);
     } else {
 #pragma unroll
       for (int ks_ = 0; ks_ < PF; ++ks_) lacc = mfma16x16x32(ones, pf[ks_], lacc);
@@ -973,15 +979,32 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
     auto exp_part = [&](const f32x16 (&s_)[NKB], V8 (&p_)[PF], int lo, int hi, bool opaque) __attribute__((always_inline)) {
       float nm = (m_run == -INFINITY) ? 0.f : kTermShift - m_run;  // fully masked row: P = 0
       if (opaque) asm("" : "+v"(nm));
+      if constexpr (TERMS == 2) {
+        // Packed pairs behind an empty asm: the lo terms read their halves (v_fma_mix) instead of
+        // converting x once more each.
 #pragma unroll
-      for (int i = 0; i < PV_STEPS; ++i)
-        if (i >= lo && i < hi)
+        for (int i = 0; i < PV_STEPS; ++i)
+          if (i >= lo && i < hi)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float x = exp2_fast(fmaf(s_[i / 2][8 * (i % 2) + j], scale_log2, nm));
-            p_[i][j] = from_f32<T>(x);
-            if constexpr (TERMS == 2) p_[PV_STEPS + i][j] = from_f32<T>(fmaf(-1.f, to_f32(p_[i][j]), x));
-          }
+            for (int j = 0; j < 8; j += 2) {
+              float x[2];
+#pragma unroll
+              for (int e = 0; e < 2; ++e) x[e] = exp2_fast(fmaf(s_[i / 2][8 * (i % 2) + j + e], scale_log2, nm));
+              f16x2 h = {(f16)x[0], (f16)x[1]};
+              asm("" : "+v"(h));
+#pragma unroll
+              for (int e = 0; e < 2; ++e) {
+                p_[i][j + e] = h[e];
+                p_[PV_STEPS + i][j + e] = (f16)fmaf(-kLoScale, (float)h[e], kLoScale * x[e]);
+              }
+            }
+      } else {
+#pragma unroll
+        for (int i = 0; i < PV_STEPS; ++i)
+          if (i >= lo && i < hi)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) p_[i][j] = from_f32<T>(exp2_fast(fmaf(s_[i / 2][8 * (i % 2) + j], scale_log2, nm)));
+      }
     };
     // S(0), its row max and the first QB P registers of a block (arrays as parameters, not
     // captures, as on the bf16 path).

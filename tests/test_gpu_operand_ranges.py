@@ -86,3 +86,38 @@ def test_fused_fp32_single_products(bh, n):
     x = (q[..., 11].abs() / 8 * 1.4427)[:, heads].unsqueeze(-1) * k[..., 11].abs()[:, heads].amax(-1)[..., None, None]
     bound = (2 * math.log(2) * 3 * 2.0 ** -24 * x + 2e-6) * v.abs().max()
     assert bool(((out - ref).abs() <= bound).all())
+
+
+def one_hot_weights(bh, n, dtype, seed, value=1.0):
+    """Integer q and k (exact dot products, scores with a standard deviation of 4) and a V that shows
+    the weights of 64 keys, spread over the row, one a dim."""
+    g = torch.Generator().manual_seed(seed)
+    q, k = (torch.randint(-3, 4, (1, bh, n, 64), generator=g).to(dtype).cuda() for _ in range(2))
+    v = torch.zeros(1, bh, n, 64, dtype=dtype, device="cuda")
+    keys = torch.arange(64, device="cuda") * n // 64
+    v[:, :, keys, torch.arange(64, device="cuda")] = value
+    return q, k, v
+
+
+@pytest.mark.parametrize("bh,n", [(2, 64), (2, 300), (300, 320), (300, 200), (140, 1000)])
+def test_fused_fp16_small_weights(bh, n):
+    """Each weight of fused with fp16 inputs (fp32 output) against float64, relative to itself: an
+    exponent of up to 64 is rounded at 2^-19 with 2^-26 of it in the scale (ln 2 of the two: 2e-6),
+    2^x, the terms and the division add 2^-22 each; below that, an absolute 2^-42 of the row's largest."""
+    q, k, v = one_hot_weights(bh, n, F16, seed=41)
+    heads = list(range(0, bh, max(1, bh // 4)))
+    out = cuda_attn.fused(q, k, v, out_dtype=F32)[:, heads].double()
+    ref = reference64(q[:, heads], k[:, heads], v[:, heads])
+    assert bool(((out - ref).abs() <= 4e-6 * ref + 2.0 ** -42).all())
+
+
+@pytest.mark.parametrize("name,bh,n", [("fused", 2, 64), ("fused", 2, 300), ("fused", 300, 320), ("fused", 140, 1000)])
+def test_fp16_small_weights_of_large_values(name, bh, n):
+    """fp16 in and out with 60000 at the key whose weight a dim shows: the products of weights down to
+    2^-41 round to what fp32 arithmetic gives: half an ulp of fp16 (2^-11 of it, 2^-25 below the normal
+    range), the weight's own error, and 60000 times an absolute 2^-43 of the row's largest weight."""
+    q, k, v = one_hot_weights(bh, n, F16, seed=43, value=60000.0)
+    heads = list(range(0, bh, max(1, bh // 4)))
+    out = getattr(cuda_attn, name)(q, k, v)[:, heads].double()
+    ref = reference64(q[:, heads], k[:, heads], v[:, heads])
+    assert bool(((out - ref).abs() <= (2.0 ** -11 + 8e-6) * ref + 2.0 ** -25 + 6e4 * 2.0 ** -43).all())
