@@ -327,8 +327,12 @@ tiled_scores_mfma(const T* __restrict__ Q, const T* __restrict__ K, float* __res
 // with the S^T blocks loaded instead of computed. A wave owns a strip of 32 query rows; per tile of BN
 // keys, the row max (m raised, and l and O rescaled, only when a row's max has outgrown it by 2^8),
 // P = 2^(S c - m), and O^T += V^T P^T on the matrix core from a V tile in LDS.
-// fp16 V: P (taken 2^7 larger, at most 2^15) as two fp16 terms, 22 bits, on the fp16 matrix core; V^T
-// read with ds_read_b64_tr_b16. fp32 V: P and V as they are on the fp32 matrix core, whose two k-slots
+// fp16 V: P (taken 2^7 larger, at most 2^15) as two fp16 terms, the lo one 2^11 larger still and with an
+// accumulator of its own, on the fp16 matrix core: 22 bits of a weight down to 2^-21 of its row's
+// largest, an absolute 2^-43 of that below, which an fp16 output does not show. (The two accumulators
+// leave three waves per SIMD at 64 dims, two past them; against one unscaled accumulator, four and three
+// waves, us: 4x16x2048 d = 64 575 -> 578, causal 391 -> 401, d = 128 676 -> 658, 1x1x4096 d = 96 58.7 -> 59.5.)
+// V^T read with ds_read_b64_tr_b16. fp32 V: P and V as they are on the fp32 matrix core, whose two k-slots
 // take the keys that the two lane halves hold.
 // V goes to LDS with direct loads (two stages), the next tile's scores to registers, during the current
 // tile; several workgroups per CU keep enough of both in flight. KS > 1: the keys are dealt tile by
@@ -336,7 +340,7 @@ tiled_scores_mfma(const T* __restrict__ Q, const T* __restrict__ K, float* __res
 // that would leave CUs without a workgroup.
 template <typename T, int NDB, int KS>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(KS == 1 && NDB <= 2 ? 4 : 3)))
+__attribute__((amdgpu_waves_per_eu(std::is_same<T, float>::value ? (KS == 1 && NDB <= 2 ? 4 : 3) : (KS == 1 && NDB == 1 ? 4 : 2))))
 tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __restrict__ O, int N, int d, float scale_log2,
                  int causal) {
   constexpr bool HALF = std::is_same<T, f16>::value;
@@ -346,7 +350,7 @@ tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __rest
   constexpr int TILE_BYTES = BN * RB, THREADS = NQ * kWave;
   constexpr int CPT = BN * CR / THREADS;            // 16-byte V chunks per thread per tile
   constexpr int NG = BN / 8;                        // groups of 4 keys per lane and tile
-  constexpr float kLazyLog2 = 8.f, kTermShift = HALF ? 7.f : 0.f;
+  constexpr float kLazyLog2 = 8.f, kTermShift = HALF ? 7.f : 0.f, kLoScale = 2048.f;
   __shared__ __attribute__((aligned(1024))) unsigned char v_lds[KS * 2 * TILE_BYTES];
   __shared__ float red_ml[KS > 1 ? (KS - 1) * 2 * kWave : 1];
   const int bh = blockIdx.y;
@@ -409,9 +413,11 @@ tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __rest
   };
 
   float m_run = -INFINITY, l_run = 0.f;
-  f32x16 o[NDB];
+  f32x16 o[NDB], o_lo[HALF ? NDB : 1];   // o_lo: the lo terms' products
 #pragma unroll
   for (int db = 0; db < NDB; ++db) o[db] = f32x16{};
+#pragma unroll
+  for (int db = 0; db < (HALF ? NDB : 1); ++db) o_lo[db] = f32x16{};
   const int kv_end = causal ? min(N, q0 + 32 * NQ) : N;
   const int ntiles = (kv_end + BN - 1) / BN, nit = (ntiles + KS - 1) / KS;
   const int wave_end = rb <= 0 ? 0 : causal ? min(N, i0 + 32) : N;   // keys that the wave's rows see
@@ -443,7 +449,10 @@ tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __rest
       m_run = raise ? m_new : m_run;
       l_run *= alpha;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) o[db] *= alpha;
+      for (int db = 0; db < NDB; ++db) {
+        o[db] *= alpha;
+        if constexpr (HALF) o_lo[db] *= alpha;
+      }
     }
     const float nm = m_run == -INFINITY ? 0.f : kTermShift - m_run;   // no visible key so far: P = 0
     float sum = 0.f;                                                  // the tile's sum, then one add to l
@@ -455,34 +464,44 @@ tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __rest
         sum += x[i][e];
       }
     l_run += sum;
+    if constexpr (HALF) {
+      // P's terms for 16 keys. (The lo terms read the packed halves of the hi ones, as in fa_mfma.hpp.)
+      auto terms = [&](int ks, f16x8& ph, f16x8& pl) __attribute__((always_inline)) {
 #pragma unroll
-    for (int ks = 0; ks < BN / 16; ++ks) {
-      if constexpr (HALF) {
-        f16x8 ph, pl;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float p = x[2 * ks + j / 4][j % 4];
-          ph[j] = (f16)p;
-          pl[j] = (f16)(p - (float)ph[j]);
+        for (int j = 0; j < 8; j += 2) {
+          const float p0 = x[2 * ks + j / 4][j % 4], p1 = x[2 * ks + j / 4][j % 4 + 1];
+          f16x2 h = {(f16)p0, (f16)p1};
+          asm("" : "+v"(h));
+          ph[j] = h[0], ph[j + 1] = h[1];
+          pl[j] = (f16)fmaf(-kLoScale, (float)h[0], kLoScale * p0);
+          pl[j + 1] = (f16)fmaf(-kLoScale, (float)h[1], kLoScale * p1);
         }
+      };
+      auto v_op = [&](int ks, int db) __attribute__((always_inline)) {
+        const unsigned char* p0 = vs + ks * 16 * RB + v_addr[db];
+        const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0));
+        const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0 + 8 * RB));
+        return __builtin_bit_cast(f16x8, i16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]});
+      };
+#pragma unroll
+      for (int ks = 0; ks < BN / 16; ++ks) {
+        f16x8 ph, pl;
+        terms(ks, ph, pl);
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
-          const unsigned char* p0 = vs + ks * 16 * RB + v_addr[db];
-          const i16x4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0));
-          const i16x4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr<i16x4>)(p0 + 8 * RB));
-          const f16x8 a = __builtin_bit_cast(f16x8, i16x8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]});
-          o[db] = mfma32x32x16(a, pl, o[db]);
+          const f16x8 a = v_op(ks, db);
+          o_lo[db] = mfma32x32x16(a, pl, o_lo[db]);
           o[db] = mfma32x32x16(a, ph, o[db]);
         }
-      } else {
-#pragma unroll
-        for (int i = 2 * ks; i < 2 * ks + 2; ++i)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int db = 0; db < NDB; ++db)
-              o[db] = mfma32x32x2(*reinterpret_cast<const float*>(vs + (8 * i + e) * RB + v_addr[db]), x[i][e], o[db]);
       }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NG; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int db = 0; db < NDB; ++db)
+            o[db] = mfma32x32x2(*reinterpret_cast<const float*>(vs + (8 * i + e) * RB + v_addr[db]), x[i][e], o[db]);
     }
   };
 
@@ -506,6 +525,11 @@ tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __rest
 #pragma unroll
     for (int i = 0; i < NG; ++i) x[i] = xn[i];
   }
+  if constexpr (HALF)
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[db][r] = fmaf(o_lo[db][r], 1.f / kLoScale, o[db][r]);
   float l = half_sum(l_run);
   if constexpr (KS > 1) {
     static_assert((KS - 1) * NDB * 16 * kWave * 4 <= KS * 2 * TILE_BYTES, "merge through the stages");

@@ -111,7 +111,8 @@ def test_fused_fp16_small_weights(bh, n):
     assert bool(((out - ref).abs() <= 4e-6 * ref + 2.0 ** -42).all())
 
 
-@pytest.mark.parametrize("name,bh,n", [("fused", 2, 64), ("fused", 2, 300), ("fused", 300, 320), ("fused", 140, 1000)])
+@pytest.mark.parametrize("name,bh,n", [("fused", 2, 64), ("fused", 2, 300), ("fused", 300, 320), ("fused", 140, 1000),
+                                       ("tiled", 2, 64), ("tiled", 3, 301), ("tiled", 64, 516), ("tiled", 140, 1000)])
 def test_fp16_small_weights_of_large_values(name, bh, n):
     """fp16 in and out with 60000 at the key whose weight a dim shows: the products of weights down to
     2^-41 round to what fp32 arithmetic gives: half an ulp of fp16 (2^-11 of it, 2^-25 below the normal
