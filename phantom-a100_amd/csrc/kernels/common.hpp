@@ -143,6 +143,50 @@ __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(f16 x) { return (float)x; }
 __device__ __forceinline__ float to_f32(bf16 x) { return (float)x; }
 
+// 32 dims of one wave's 32 rows of O again in plain fp32 FMAs, for rows of which the matrix core's result
+// has an element that is not finite (an infinity in V times a 16-bit term or a masked weight of zero is a
+// NaN; a sum of weights not yet normalised can overflow): acc = sum over keys < `keys` of the key's weight
+// times V[key], in an accumulator's layout (register r: dim c0 + 8 (r / 4) + 4 (lane / 32) + r % 4 of
+// query lane % 32). weights(k0, p), called by all lanes, gives the fp32 weights of keys k0 ..
+// k0 + KEYS - 1 in the lane's row, negative where the row does not see the key. Rows of V are d elements,
+// whole groups of four and aligned to them. (KEYS keys' loads are in flight together: one at a time, the
+// loop waits ~1.2 us a key.)
+template <int KEYS, typename T, typename Weights>
+__device__ __forceinline__ void retake_rows(f32x16& acc, const T* V, int d, int c0, int keys, Weights weights) {
+  typedef T T4 __attribute__((ext_vector_type(4)));
+  int off[4];   // (dims past d, which are not stored, take the row's first ones)
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    off[g] = c0 + 8 * g + 4 * ((int)threadIdx.x % kWave / 32);
+    off[g] = off[g] < d ? off[g] : 0;
+  }
+  acc = f32x16{};
+#pragma unroll 1
+  for (int k0 = 0; k0 < keys; k0 += KEYS) {
+    float p[KEYS];
+    weights(k0, p);
+    T4 v[KEYS][4];
+#pragma unroll
+    for (int k = 0; k < KEYS; ++k)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        v[k][g] = *reinterpret_cast<const T4*>(V + (size_t)min(k0 + k, keys - 1) * d + off[g]);
+#pragma unroll
+    for (int k = 0; k < KEYS; ++k)
+      if (k0 + k < keys && !(p[k] < 0.f)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = fmaf(p[k], to_f32(v[k][r / 4][r % 4]), acc[r]);
+      }
+  }
+}
+// Whether a lane's accumulator holds an element that is not finite.
+__device__ __forceinline__ bool any_not_finite(const f32x16& o) {
+  float z = 0.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) z = fmaf(o[r], 0.f, z);
+  return z != 0.f;   // 0, or a NaN
+}
+
 // Maps the hardware workgroup id to a logical one so that consecutive logical ids run on the
 // same XCD: the dispatcher sends workgroup g to XCD g % 8, so logical id
 // (g % 8) * (total / 8) + g / 8 keeps a contiguous range of (head, query-block) pairs - the

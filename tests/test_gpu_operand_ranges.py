@@ -88,6 +88,45 @@ def test_fused_fp32_single_products(bh, n):
     assert bool(((out - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("bh,n,d", [(1, 2, 64), (3, 333, 40), (2, 130, 128), (70, 515, 64), (40, 901, 96)])
+def test_tiled_fp32_largest_values(bh, n, d, causal):
+    """Values near the largest float, which a sum of unnormalised weights would carry to infinity."""
+    q, k, v = make_qkv(1, bh, n, d, F32, seed=29, device="cuda")
+    v = 3.2e38 * (1 - 0.05 * v.abs().clamp(max=10) / 10) * torch.where(torch.arange(d, device="cuda") % 3 == 0, -1.0, 1.0)
+    v[..., 1] = torch.randn(v.shape[:-1], device="cuda", generator=torch.Generator("cuda").manual_seed(3))
+    heads = list(range(0, bh, max(1, bh // 4)))
+    out = cuda_attn.tiled(q, k, v, causal)[:, heads].double()
+    ref = reference64(q[:, heads], k[:, heads], v[:, heads], causal)
+    big = torch.arange(d, device="cuda") != 1
+    assert bool(((out - ref)[..., big].abs() <= 4e-6 * ref[..., big].abs()).all())
+    assert bool(((out - ref)[..., 1].abs() <= 1e-5).all())
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dtype", [F32])
+@pytest.mark.parametrize("bh,n,d", [(2, 37, 40), (2, 300, 64), (3, 301, 80), (2, 131, 128), (64, 515, 64), (64, 514, 40),
+                                    (64, 513, 128)])
+def test_tiled_infinite_values(bh, n, d, dtype, causal):
+    """An infinite element of V is infinite in its dim of the rows that see it, a NaN is NaN there, and
+    nothing else is touched."""
+    q, k, v = make_qkv(1, bh, n, d, dtype, seed=31, device="cuda")
+    places = {(0, n // 2, 5): INF, (0, n // 3, 7): -INF, (bh - 1, n - 1, 33): INF, (bh - 1, 2, 34): float("nan")}
+    zeroed = v.clone()
+    for (h, key, c), x in places.items():
+        v[0, h, key, c], zeroed[0, h, key, c] = x, 0
+    out, want = cuda_attn.tiled(q, k, v, causal), cuda_attn.tiled(q, k, zeroed, causal)
+    rows = torch.arange(n, device="cuda")
+    keep = torch.ones_like(out, dtype=torch.bool)
+    for (h, key, c), x in places.items():
+        sees = rows >= key if causal else rows >= 0
+        got = out[0, h, sees, c]
+        assert bool(got.isnan().all() if math.isnan(x) else (got == x).all())
+        keep[0, h, sees, c] = False
+    bar = 1e-5 if dtype == F32 else 2e-3
+    assert bool(((out - want).abs()[keep] <= bar).all())
+
+
 def one_hot_weights(bh, n, dtype, seed, value=1.0):
     """Integer q and k (exact dot products, scores with a standard deviation of 4) and a V that shows
     the weights of 64 keys, spread over the row, one a dim."""
