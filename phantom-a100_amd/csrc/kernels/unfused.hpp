@@ -566,7 +566,7 @@ tiled_softmax_pv(const float* __restrict__ S, const T* __restrict__ V, T* __rest
   const float inv = 1.f / l;
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
-    if (!HALF && __builtin_amdgcn_ballot_w64(qrow < N && any_not_finite(o[db]) && __builtin_isfinite(l)) != 0) {
+    if (__builtin_amdgcn_ballot_w64(qrow < N && any_not_finite(o[db]) && __builtin_isfinite(l)) != 0) {
       constexpr int KEYS = HALF ? 8 : KS == 1 && NDB <= 2 ? 2 : 4;   // (what the registers hold)
       f32x16 acc;
       retake_rows<KEYS>(acc, V + (size_t)bh * N * d, d, 32 * db, wave_end, [&](int k0, float (&p)[KEYS]) __attribute__((always_inline)) {

@@ -104,7 +104,7 @@ def test_tiled_fp32_largest_values(bh, n, d, causal):
 
 
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("dtype", [F32])
+@pytest.mark.parametrize("dtype", [F16, F32])
 @pytest.mark.parametrize("bh,n,d", [(2, 37, 40), (2, 300, 64), (3, 301, 80), (2, 131, 128), (64, 515, 64), (64, 514, 40),
                                     (64, 513, 128)])
 def test_tiled_infinite_values(bh, n, d, dtype, causal):
