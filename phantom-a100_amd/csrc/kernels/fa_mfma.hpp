@@ -345,8 +345,8 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
     for (int j = 0; j < 8; ++j) ones[j] = from_f32<T>(on ? 1.f : 0.f);
   }
   f32x16 o[NDB];
-  // TERMS == 2: the lo terms' products, summed apart (half the roundings at the size of O, and an
-  // infinite V meets a lo term of either sign without turning O into a NaN) and added at the end.
+  // TERMS == 2: the lo terms' products, summed apart (half the roundings at the size of O, and their
+  // own scale) and added at the end.
   f32x16 o_lo[TERMS == 2 ? NDB : 1];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
@@ -358,7 +358,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] = __builtin_isfinite(o[db][r]) ? fmaf(o_lo[db][r], 1.f / kLoScale, o[db][r]) : o[db][r];
+        for (int r = 0; r < 16; ++r) o[db][r] = fmaf(o_lo[db][r], 1.f / kLoScale, o[db][r]);
   };
 
   const int kv_end = causal ? min(N, q0 + BM) : N;
@@ -554,7 +554,40 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
       if (p + 1 < PASSES) __builtin_amdgcn_s_waitcnt(0xc07f);   // reads done before the next pass
     }
   };
+  // TERMS == 2: rows with an element that is not finite again with fp32 weights (an infinity in V times
+  // a term of zero is a NaN). The scores again too, each lane half taking half of the dims.
+  auto retake = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+      if (__builtin_amdgcn_ballot_w64(qrow < N && any_not_finite(o[db]) && __builtin_isfinite(lacc[0])) != 0) {
+        constexpr int KEYS = 2;   // (4 keys' operands crowd the main loop's registers)
+        const int keys = causal ? min(N, q0w + 32) : N;
+        const T* qp = Q + base + (size_t)min(qrow, N - 1) * D + hi * (D / 2);
+        const float nm = kTermShift - m_run;
+        f32x16 acc;
+        retake_rows<KEYS>(acc, V + base, D, 32 * db, keys, [&](int k0, float (&p)[KEYS]) __attribute__((always_inline)) {
+#pragma unroll
+          for (int k = 0; k < KEYS; ++k) {
+            const int key = min(k0 + k, keys - 1);
+            const T* kp = K + base + (size_t)key * D + hi * (D / 2);
+            float dot = 0.f;
+#pragma unroll
+            for (int c = 0; c < D / 2; c += 8) {
+              const V8 a = *reinterpret_cast<const V8*>(qp + c), b = *reinterpret_cast<const V8*>(kp + c);
+#pragma unroll
+              for (int j = 0; j < 8; ++j) dot = fmaf((float)a[j], (float)b[j], dot);
+            }
+            p[k] = exp2_fast(fmaf(half_sum(dot), scale_log2, nm));
+            if (causal && key > qrow) p[k] = -1.f;
+          }
+        });
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] = __builtin_isfinite(o[db][r]) ? o[db][r] : acc[r];
+      }
+  };
   auto store_block = [&]() {
+    if constexpr (TERMS == 2)
+      if (g == 0) retake();
     if constexpr (PERSIST) {
       store_rows(o_lds + wave * ORW * OROW, std::integral_constant<int, ORW>{});
     } else if constexpr (PB_STAGED) {
@@ -1248,6 +1281,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
       const float sc0 = (m_out == -INFINITY) ? 0.f : exp2_fast(m_out - m);
       const float sc1 = (m1 == -INFINITY) ? 0.f : exp2_fast(m1 - m);
       lacc = sc0 * lacc + sc1 * l1;
+      if constexpr (TERMS == 2) m_run = m;   // (the rows' own, if they are taken again)
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll

@@ -127,6 +127,42 @@ def test_tiled_infinite_values(bh, n, d, dtype, causal):
     assert bool(((out - want).abs()[keep] <= bar).all())
 
 
+# Key split, persistent with whole and ragged last tiles, one tile a row.
+FUSED_F16_GRIDS = [(2, 300), (300, 320), (300, 200), (140, 1000), (3, 64), (300, 40)]
+
+
+@pytest.mark.parametrize("out_dtype", [F16, F32])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("bh,n", FUSED_F16_GRIDS)
+def test_fused_fp16_infinite_value_of_small_weight(bh, n, causal, out_dtype):
+    """An infinite element of V whose key has a weight of e^-50 (any positive fp32 weight makes it
+    infinite), in the key groups and launch forms of fused with fp16 inputs."""
+    q, k, v = make_qkv(1, bh, n, 64, F16, seed=37, device="cuda")
+    q[..., 0] = 1
+    j = min(17, n - 2)
+    k[..., 0] = 0
+    k[..., j, :] = 0
+    k[..., j, 0] = -400
+    want = cuda_attn.fused(q, k, v, causal, out_dtype=out_dtype)
+    v[0, 0, j, 5] = INF
+    v[0, bh - 1, j, 63] = -INF
+    rows = torch.arange(n, device="cuda")
+    sees = rows > j if causal else rows >= 0
+    for persistent in (True, False):
+        prev = _native.set_persistent(persistent)
+        try:
+            out = cuda_attn.fused(q, k, v, causal, out_dtype=out_dtype)
+        finally:
+            _native.set_persistent(prev)
+        assert bool((out[0, 0, sees, 5] == INF).all() and (out[0, bh - 1, sees, 63] == -INF).all())
+        keep = torch.ones_like(out, dtype=torch.bool)
+        keep[0, 0, :, 5] = keep[0, bh - 1, :, 63] = False
+        same = torch.equal(out[keep], want[keep])
+        assert same
+        hidden = rows < j if causal else rows < 0
+        assert bool(((out - want)[:, :, hidden].abs() <= 2e-3).all())
+
+
 def one_hot_weights(bh, n, dtype, seed, value=1.0):
     """Integer q and k (exact dot products, scores with a standard deviation of 4) and a V that shows
     the weights of 64 keys, spread over the row, one a dim."""
