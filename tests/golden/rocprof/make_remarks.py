@@ -24,10 +24,10 @@ PKG = os.path.join(REPO, "phantom-a100_amd")
 # kernel (bf16 d=128, BM=256), a one-stage fused_tuned tile and the fp32 fused kernel.
 KERNELS = [
     "_ZN2pa13naive_softmaxE",
-    "_ZN2pa11fa_mfma_fwdIDF16_Li64ELi128ELi64ELi2EfLi1ELb1ELb0ELb0ELb1EEEv",
-    "_ZN2pa11fa_mfma_fwdIDF16bLi128ELi256ELi64ELi2EDF16bLi1ELb1ELb0ELb0ELb0EEEv",
-    "_ZN2pa11fa_mfma_fwdIDF16_Li64ELi128ELi32ELi1EDF16_Li1ELb0ELb0ELb0ELb0EEEv",
-    "_ZN2pa10fa_f32_fwdIfLi64ELi4EfEEv",
+    "_ZN2pa11fa_mfma_fwdIDF16_Li64ELi128ELi64ELi2EfLi1ELb1ELb0ELb0ELb1ELi1EEEv",
+    "_ZN2pa11fa_mfma_fwdIDF16bLi128ELi256ELi64ELi2EDF16bLi1ELb1ELb0ELb0ELb0ELi1EEEv",
+    "_ZN2pa11fa_mfma_fwdIDF16_Li64ELi128ELi32ELi1EDF16_Li1ELb0ELb0ELb0ELb0ELi1EEEv",
+    "_ZN2pa10fa_f32_fwdILi64ELi4EEEv",
 ]
 
 

@@ -5,6 +5,7 @@ the bottleneck rules. The GPU runs of the same tools are in test_gpu_tools.py.""
 from __future__ import annotations
 
 import importlib.util
+import json
 import os
 import re
 import sys
@@ -315,6 +316,21 @@ def test_parse_resource_remarks():
     # 64 KB of K/V stages and 64 KB of O staging rows
     assert c4["vgprs"] == 224 and c4["agprs"] == 0 and c4["lds_bytes"] == 131072
     assert c4["occupancy_waves_per_simd"] == 2 and c4["vgpr_spill"] == 0 and c4["scratch_bytes"] == 0
+
+
+def test_remarks_generator_names_current_kernels():
+    """Every kernel that the fixture's generator names is in the fixture, and is one kernel of the built
+    library: a change of a kernel's template arguments reaches the generator too."""
+    spec = importlib.util.spec_from_file_location("make_remarks", os.path.join(FIX, "make_remarks.py"))
+    gen = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(gen)
+    sets = [resources_fixture()]
+    if os.path.exists(build_native.RESOURCES):
+        with open(build_native.RESOURCES) as fh:
+            sets.append(json.load(fh))
+    for res in sets:
+        for prefix in gen.KERNELS:
+            assert sum(name.startswith(prefix) for name in res) == 1, prefix
 
 
 def test_vgpr_occupancy_model_agrees_with_the_compiler():
