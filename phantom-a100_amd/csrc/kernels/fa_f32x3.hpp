@@ -18,10 +18,11 @@
 // four query waves walk alternate tiles and are merged at the end, which gives a CU its two waves per
 // SIMD from one workgroup.
 //
-// Measured: 4x16x2048 601 -> 379 us (114 -> 181 TFLOP/s), 4x16x4096 2322 -> 1464 us (188), causal
-// 4x16x1024 114 -> 62 us, 2x4x4000 292 -> 185 us (177). At those sizes the six products run at
-// ~1.1 PFLOP/s of bf16 matrix work, about what a large bf16 product reaches under the card's power
-// cap; interleaving the staging with the products by scheduling groups, or a raised wave priority
+// Measured, us a call: 4x16x2048 607 -> 393 (113 -> 175 TFLOP/s), 4x16x4096 2320 -> 1475 (186), causal
+// 4x16x1024 114 -> 62, 2x4x4000 293 -> 179. At those sizes the six products run at ~1.1 PFLOP/s of bf16
+// matrix work, about what a large bf16 product reaches under the card's power cap. Counters at
+// 4x16x2048: matrix core busy 52 % of the cycles, VALU 58 %, a VALU instruction beside 35 % of the MFMA
+// cycles; interleaving the staging with the products by scheduling groups, or a raised wave priority
 // for them, moved nothing (within 1 %), three waves per SIMD spill (146 VGPRs, 8 % slower), and
 // keeping each wave's own tiles in registers (no LDS, as fa_f32.hpp) loses 5 % to fa_f32.hpp because
 // every wave then splits its operands itself.

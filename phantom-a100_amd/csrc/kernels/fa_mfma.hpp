@@ -1100,7 +1100,7 @@ fa_mfma_fwd(const T* __restrict__ Q, const T* __restrict__ K, const T* __restric
             // (the fused_tc d = 64 tile measured fastest at 4 and, in phase B, 8: C3 +0.5 %,
             // C5 +0.6 % over the per-phase totals 5 and 11, within 1 % for 4-6 and 4-11)
             constexpr int VA = TERMS == 2 ? 8 : (D == 64 && BM == 128 && BN == 64 && !RS)
-                                   ? 4 : ((PV_STEPS - QB) * 20 + (RS ? NDB * 16 * TERMS + 2 : 0) + QK_MFMAS - 1) / QK_MFMAS;
+                                   ? 4 : ((PV_STEPS - QB) * 20 + (RS ? NDB * 16 + 2 : 0) + QK_MFMAS - 1) / QK_MFMAS;
             // Phase A at wave priority 2, as on the bf16 path (causal fp16 d = 64 4x16x1024 +2.1-3.1 %,
             // 1x16x2048 +1.0-1.2 %); not in the key split, which lost 8 % with it (C2, 1x4x8192).
             if constexpr (KSPLIT == 1) __builtin_amdgcn_s_setprio(2);

@@ -16,7 +16,7 @@
 #pragma once
 
 #include "common.hpp"
-#include "fa_mfma.hpp"   // v_swz: the V tile layout of the fused kernel, reused by tiled_pv_mfma
+#include "fa_mfma.hpp"   // v_swz: the V tile layout of the fused kernel, reused by tiled_softmax_pv
 
 namespace pa {
 
@@ -27,8 +27,8 @@ namespace pa {
 // rows, P rows) is the same address in every lane, and the per-lane operand (a K row, a V column)
 // serves R rows. One row per wave spent an L1 access on every FMA (a lane's K row piece, a V element);
 // with the rows' operands in scalar registers, R FMAs share it, and what is left is the latency of
-// the loads, issued 16 elements at a time: fp32 2x8x333 d = 80 300 -> 56 us, fp32 8x16x1024 d = 128
-// 19.8 -> 2.3 ms, fp16 324x128 d = 64 223 -> 74 us, fp32 42x128 53 -> 23 us, same bits. Grids are
+// the loads, issued 16 elements at a time: fp32 2x8x333 d = 80 298 -> 56 us, fp32 8x16x1024 d = 128
+// 19.8 -> 2.3 ms, fp16 324x128 d = 64 232 -> 78 us, fp32 42x128 52 -> 19 us, same bits. Grids are
 // flattened into x: row groups times column blocks.
 
 // S[h][i][j0 + lane] for the wave's R query rows i and 64 keys from j0; keys after i are -inf when
@@ -221,25 +221,25 @@ tiled_scores(const T* __restrict__ Q, const T* __restrict__ K, float* __restrict
 // its P^T operands the same way. (A strip starts 16-byte aligned only where N * N * head does: the
 // vectors are declared with an element's alignment.)
 //
-// Measured, three kernels -> two, us: fp16 4x16x2048 d = 64 980 -> 580 (scores 286, the rest 279: 3.8
-// TB/s each), causal 942 -> 394, 4x8x4096 1787 -> 945, 8x32x256 59 -> 39; fp32 4x16x2048 1350 -> 791
-// (both kernels also near the fp32 matrix core's rate). Rows and head dims that took the VALU kernels:
-// fp16 1x8x2000 d = 80 408 -> 63, 2x32x2047 d = 32 2022 -> 476, 1x1x4096 d = 96 641 -> 60; fp32
-// 1x16x333 d = 40 92 -> 20. Passes over a few heads at a time, whose scores stay in the memory-side
+// Measured, three kernels -> two, us a call: fp16 4x16x2048 d = 64 983 -> 561, causal 922 -> 405, 4x8x4096
+// 1771 -> 919, 8x32x256 58 -> 38 (4x16x4096: the scores stored at 3.9 TB/s, read at 5.1); fp32 4x16x2048
+// 1327 -> 758 (both kernels also near the fp32 matrix core's rate). Rows and head dims that took the VALU
+// kernels: fp16 1x8x2000 d = 80 407 -> 61, 2x32x2047 d = 32 2022 -> 468, 1x1x4096 d = 96 640 -> 60; fp32
+// 1x16x333 d = 40 91 -> 20. Passes over a few heads at a time, whose scores stay in the memory-side
 // cache (192 MiB), gained 8 % at 4x16x2048 but lost up to 20 % on causal rows and smaller grids.
-// Against float64 the error is no larger (fp32 1x5x3392 d = 128 causal 5.2e-7 -> 3.8e-7; fp16 its
-// output's rounding).
+// Against float64 (2-norms) the error is no larger on N(0, 1) inputs (fp32 1x5x3392 d = 128 causal 5.2e-7
+// -> 3.8e-7; fp16 its output's rounding) and within 1.4 % with q and k times 3, where the scores' own
+// roundings set it; the largest element's error falls there as often as it grows.
 typedef float Score4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// Operands of an S^T = K Q^T block for the matrix core, read straight from memory in the MFMA layout;
-// rows past N and dims past d read as zero through the buffer's range.
-// fp16: one 32x32x16 step takes dims 16 kk + 8 (l / 32) .. + 7 of row l % 32.
-// fp32: 16 steps of 32x32x2 take dims 16 (l / 32) + 0 .. 15 of a 32-dim chunk, in Q and K alike.
 constexpr uint32_t kNoRow = 0x80000000u;   // an offset past every head (a head is below 2 GiB)
 
 // S^T blocks of 128 queries x 128 keys per workgroup, 64 x 64 per wave as 2 x 2 blocks of 32 x 32.
 // With causal, blocks whose keys all come after their queries are neither computed nor stored (the
-// second kernel does not read them).
+// second kernel does not read them). The operands are read straight from memory in the MFMA layout; rows
+// past N and dims past d read as zero through the buffer's range. fp16: one 32x32x16 step takes dims
+// 16 kk + 8 (l / 32) .. + 7 of row l % 32. fp32: 16 steps of 32x32x2 take dims 16 (l / 32) + 0 .. 15 of a
+// 32-dim chunk, in Q and K alike.
 template <typename T>
 __global__ void __launch_bounds__(256)
 tiled_scores_mfma(const T* __restrict__ Q, const T* __restrict__ K, float* __restrict__ S, int N, int d, int causal) {

@@ -360,7 +360,7 @@ const MfmaEntry* find_tuned(int dtype, int out_dtype, int64_t d, int br, int bc,
 }
 
 // ------------------------------------------------------------------ fused, fp32 arithmetic
-// fp32 inputs, three kernels. fa_f32_fwd (fp32 matrix core): 32 query rows per workgroup, keys split
+// fp32 inputs, two kernels. fa_f32_fwd (fp32 matrix core): 32 query rows per workgroup, keys split
 // over kF32KS waves. fa_f32x3_fwd (bf16 matrix core, three-term operands): 128 query rows per
 // workgroup, in one key group of 4 waves or two of them.
 constexpr int kF32KS = 4;
@@ -417,9 +417,9 @@ hipError_t launch_f16_terms(const void* q, const void* k, const void* v, void* o
 // ------------------------------------------------------------------ unfused
 // Query rows a wave of a naive product takes: 8, which reuse each K / V element 8 times, where that
 // still leaves a wave for each of the chip's 1024 SIMDs, else 2 (a wave is then bound by its loads'
-// latency, and more of them run at once). Measured at 2 / 8 rows, us: fp32 8x16x1024 d = 128 5180 /
-// 2271, fp16 4x16x512 281 / 202, fp32 42x128 23.6 / 26.3, fp16 causal 2x600 d = 96 32 / 87; 4 rows lay
-// between the two, 16 were slower than 8.
+// latency, and more of them run at once). Measured with both products at 2 / 8 rows, us: fp32 8x16x1024
+// d = 128 5180 / 2271, fp16 4x16x512 281 / 202, fp32 42x128 23.6 / 26.3 (18.7 as the rule has it: scores
+// at 8, P.V at 2), fp16 causal 2x600 d = 96 32 / 87; 4 rows lay between the two, 16 were slower than 8.
 int naive_rows(long long n, long long col_blocks, long long bh) {
   return (n + 7) / 8 * col_blocks * bh >= 4 * kCUs ? 8 : 2;
 }

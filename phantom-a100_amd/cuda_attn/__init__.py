@@ -97,7 +97,7 @@ def _unfused(fn_name: str, err_name: str, q, k, v, causal: bool) -> torch.Tensor
 
 
 def naive(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = False) -> torch.Tensor:
-    """v1: three kernels, one thread per output, N x N scores in HBM."""
+    """v1: three kernels of plain loops, a few query rows per wave, N x N scores in HBM."""
     return _unfused("pa_naive_fwd", "naive_forward", q, k, v, causal)
 
 

@@ -93,7 +93,7 @@ def fused_tc_kernel(dtype: int, out_dtype: int, bh: int, n: int, d: int, causal:
 
 
 def set_persistent(enable: bool) -> bool:
-    """Switch fused_tc's persistent launch on or off (every shape that would take it: causal calls,
+    """Switch the persistent launch of fused_tc, and of fused with fp16 inputs, on or off (every shape that would take it: causal calls,
     and non-causal ones with an even number of 64-key tiles or an odd number, above one, of full
     ones, at d = 64 and 128); returns the previous setting. fused_tc_kernel names the launch."""
     return bool(lib().pa_set_persistent(int(bool(enable))))

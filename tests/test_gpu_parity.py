@@ -201,10 +201,9 @@ def test_other_head_dims_for_unfused(name, d, causal):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("causal", [False, True])
 def test_naive_piece_loads_match_element_loads(dtype, causal):
-    """naive reads Q and K rows a 16-byte piece per load when they are 16-byte aligned and hold
-    whole pieces, and the P rows four probabilities per load when the workspace is aligned and
-    N % 4 == 0; otherwise an element per load. The products are summed in the same order either
-    way, so inputs (and a workspace) one element off alignment give the same bits."""
+    """naive reads K rows a 16-byte piece per load when they are 16-byte aligned and hold whole
+    pieces, otherwise an element per load. The products are summed in the same order either way, so
+    inputs (and a workspace) one element off alignment give the same bits."""
     b, h, n, d = 1, 3, 260, 64
     code = {torch.float32: _native.DTYPE_F32, torch.float16: _native.DTYPE_F16}[dtype]
     q, k, v = make_qkv(b, h, n, d, dtype, seed=9, device="cuda")
@@ -489,8 +488,8 @@ def test_fused_fp16_inputs_keep_fp32_arithmetic(bh, n, causal):
 
 
 def test_fused_fp16_infinite_value_stays_infinite():
-    """An infinite element of V gives an infinite (not NaN) output in its dim where its weight is not
-    tiny, as a product with an fp32 weight does; the other dims are not touched."""
+    """An infinite element of V gives an infinite (not NaN) output in its dim, as a product with an
+    fp32 weight does; the other dims are not touched."""
     q, k, v = gpu_qkv(1, 2, 300, 64, torch.float16, seed=7)
     want = cuda_attn.fused(q, k, v, out_dtype=torch.float32)
     v[0, 0, 17, 5] = float("inf")
